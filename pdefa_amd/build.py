@@ -29,6 +29,7 @@ SOURCES = [
     "kernels/conv_wino.hip",
     "kernels/conv_wino_strip.hip",
     "kernels/ops.hip",
+    "kernels/relayout.hip",
     "kernels/yolo_decode.hip",
     "kernels/noalloc.hip",
     "model.cpp",

@@ -140,6 +140,10 @@ struct ConvArgs {
     const float* w_kmaj = nullptr;
     float jump_window = 1.52587890625e-05f;
     int32_t KH = 1, KW = 1, sh = 1, sw = 1, ph = 0, pw = 0, dh = 1, dw = 1;
+    // first output row: the launch computes rows [row0, row0 + Ho) of the
+    // image's output, y (and res) pointing at row row0 (the launchers pass
+    // the kernels ph - row0 * sh, the padding seen from that row)
+    int32_t row0 = 0;
     int32_t K = 0;        // KH*KW*Cin
     int32_t ktiles = 0;   // ceil(K / 32): 32-wide K blocks of the packed weights
     int32_t act = 0;
@@ -296,6 +300,25 @@ enum EltOp : int32_t {
 };
 void launch_eltwise(int op, const View& out, const View& a, const View& b, float alpha,
                     hipStream_t s);
+
+// A planar [N][C][P] tensor (P contiguous pixels per channel: NCHW) and its
+// channels-last form [N][P][C] (C contiguous channels per pixel), either of
+// which may be page-locked host memory; see kernels/relayout.hip.
+constexpr int kTransferBlocks = 128;  // workgroups of a kernel on host memory
+struct RelayoutArgs {
+    const float* src = nullptr;
+    float* dst = nullptr;
+    float* mirror = nullptr;  // rows to planar: optional second copy of dst
+    bool host = false;        // one side is host memory
+    int32_t N = 0, C = 0, P = 0;
+    int64_t planar_n = 0, planar_c = 0;  // strides of the planar side
+    int64_t rows_n = 0, rows_p = 0;      // strides of the channels-last side
+};
+void launch_planar_to_rows(const RelayoutArgs& a, hipStream_t s);
+void launch_rows_to_planar(const RelayoutArgs& a, hipStream_t s);
+// n contiguous floats between 16-byte aligned addresses, either of which may
+// be page-locked host memory.
+void launch_copy_floats(float* dst, const float* src, int64_t n, hipStream_t s);
 
 // Max pooling over logical [N, C, H, W] views (padding never wins).
 void launch_maxpool(const View& out, const View& in, int kh, int kw, int sh, int sw, int ph,

@@ -198,6 +198,8 @@ void check_conv(const ConvArgs& a, const ConvTileShape& sh, bool vec) {
     if (a.ktiles != (a.K + BK - 1) / BK) fail("ktiles mismatch");
     const int64_t M = static_cast<int64_t>(a.N) * a.Ho * a.Wo;
     if (a.groups < 1) fail("groups < 1");
+    if (a.row0 < 0 || a.row0 + static_cast<int64_t>(a.Ho) >= (int64_t{1} << 24)) fail("output rows");
+    if (a.row0 > 0 && a.splits != 1) fail("split-K takes whole images");
     if (M * std::max(a.Cout, 1) * a.groups >= (int64_t{1} << 31)) fail("M * Cout too large");
     if (a.groups > 1 && a.w_group < packed_weight_elems(a.Cout, a.K)) fail("packed weights per group too small");
     if (a.splits < 1 || a.kt_per_split < 1 || a.kt_per_split % sh.kg != 0 ||
@@ -219,9 +221,10 @@ void check_conv(const ConvArgs& a, const ConvTileShape& sh, bool vec) {
 }
 
 // The problem's divisors for the kernel's index arithmetic (every one below
-// 2^31: check_conv bounds the extents).
+// 2^31: check_conv bounds the extents), and its padding seen from row0.
 ConvArgs with_divisors(const ConvArgs& a) {
     ConvArgs b = a;
+    b.ph = a.ph - a.row0 * a.sh;
     b.fd_howo = make_fastdiv(static_cast<int64_t>(a.Ho) * a.Wo);
     b.fd_wo = make_fastdiv(a.Wo);
     b.fd_cin = make_fastdiv(a.Cin);

@@ -1744,6 +1744,14 @@ class Planner {
             plan_.bufs[o.buf].first = std::min(plan_.bufs[o.buf].first, n);
             plan_.bufs[o.buf].last = n;
         }
+        if (opt_.pin_io && n >= 2)
+            for (const Step* s : {&plan_.steps.front(), &plan_.steps.back()})
+                if (s->kind == StepKind::Elt && s->elt == k::kEltCopy)
+                    for (int32_t b : {s->a.buf, s->out.buf})
+                        if (b >= 0) {
+                            plan_.bufs[b].first = -1;
+                            plan_.bufs[b].last = n;
+                        }
         // Greedy by size: each buffer takes the lowest 256-byte aligned offset that
         // does not overlap a live-range-overlapping buffer already placed.
         std::vector<int> order(plan_.bufs.size());

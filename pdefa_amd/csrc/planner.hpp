@@ -141,6 +141,10 @@ struct PlanOptions {
     // > 0: Plan::early_steps covers the leading per-image steps whose outputs
     // have at least this many pixels (H * W)
     int64_t early_hw = 0;
+    // The program's first layout copy (of an input) and last one (of an
+    // output) may run as transfers that overlap other steps: the memory they
+    // touch is shared with nothing.
+    bool pin_io = false;
 };
 
 // Throws std::runtime_error naming the node for an unsupported op or pattern.

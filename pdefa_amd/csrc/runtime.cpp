@@ -401,6 +401,9 @@ Session::Session(Model& m) : model_(&m) {
     // it lands; PDEFA_EARLY_HW: the smallest output map (H * W) of an early step
     if (const char* c = std::getenv("PDEFA_INPUT_CHUNKS")) input_chunks_ = std::atoi(c);
     if (const char* h = std::getenv("PDEFA_EARLY_HW")) early_hw_ = std::atoll(h);
+    // PDEFA_IO_SLICES=n: cut a program between layout copies into at most n
+    // slices (1: none)
+    if (const char* c = std::getenv("PDEFA_IO_SLICES")) io_slices_ = std::max(0, std::atoi(c));
     opts_.split_k = env_flag("PDEFA_SPLITK", true);
     if (const char* t = std::getenv("PDEFA_CONV_TILE")) {
         for (int i = 0; i < k::kNumConvShapes; ++i)
@@ -606,6 +609,12 @@ Session::Prepared::~Prepared() {
         if (g.graph) (void)hipGraphDestroy(g.graph);
         if (g.done) (void)hipEventDestroy(g.done);
     }
+    for (IoSlice& c : io) {
+        if (c.exec) (void)hipGraphExecDestroy(c.exec);
+        if (c.graph) (void)hipGraphDestroy(c.graph);
+        if (c.pulled) (void)hipEventDestroy(c.pulled);
+        if (c.computed) (void)hipEventDestroy(c.computed);
+    }
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     for (hipEvent_t e : events)
@@ -672,6 +681,7 @@ void Session::prepare(const std::vector<std::vector<int64_t>>& dims) {
                      batch % chunks == 0)
                         ? early_hw_
                         : 0;
+    opts.pin_io = use_graph_ && !concurrent_;
     if (autotune_) {
         opts.tune_conv = [this](const ConvQuery& q) { return tune_conv(q, stream_); };
         // grouped launches change the program order; the concurrent capture
@@ -946,7 +956,12 @@ void Session::prepare(const std::vector<std::vector<int64_t>>& dims) {
     }
     plan_input_chunks();
     plan_segments();
+    plan_io();
 }
+
+// Launch lists up to this long are issued one by one: a graph launch costs
+// the host about as much.
+static constexpr size_t kGraphLaunches = 3;
 
 void Session::launch_one(const Launch& l, hipStream_t s) {
     switch (l.kind) {
@@ -1282,6 +1297,321 @@ void Session::run_segments() {
     if (copy_in_) PDEFA_HIP(hipStreamSynchronize(copy_in_));
 }
 
+namespace {
+
+// A dense row-major rank-4 [N, C, H, W] view.
+bool dense4(const k::View& v) {
+    return v.rank == 4 && v.str[3] == 1 && v.str[2] == v.dims[3] && v.str[1] == v.dims[2] * v.dims[3] &&
+           v.str[0] == v.dims[1] * v.str[1];
+}
+// A channels-last one whose pixels follow each other evenly.
+bool rows4(const k::View& v) {
+    return v.rank == 4 && v.str[1] == 1 && v.str[3] >= v.dims[1] && v.str[2] == v.dims[3] * v.str[3] && v.str[0] >= 0;
+}
+bool same_dims(const k::View& a, const k::View& b) {
+    if (a.rank != b.rank) return false;
+    for (int d = 0; d < a.rank; ++d)
+        if (a.dims[d] != b.dims[d]) return false;
+    return true;
+}
+
+// Pixels [p0, p0 + P) of images [n0, n0 + N) of a planar/channels-last pair.
+k::RelayoutArgs relayout_of(const k::View& planar, const k::View& rows, int64_t n0, int64_t N, int64_t p0, int64_t P,
+                            bool to_rows) {
+    k::RelayoutArgs r;
+    r.N = static_cast<int32_t>(N);
+    r.C = static_cast<int32_t>(planar.dims[1]);
+    r.P = static_cast<int32_t>(P);
+    r.planar_n = planar.str[0];
+    r.planar_c = planar.str[1];
+    r.rows_n = rows.str[0];
+    r.rows_p = rows.str[3];
+    float* p = planar.ptr + n0 * planar.str[0] + p0;
+    float* q = rows.ptr + n0 * rows.str[0] + p0 * rows.str[3];
+    r.src = to_rows ? p : q;
+    r.dst = to_rows ? q : p;
+    return r;
+}
+
+}  // namespace
+
+// Microseconds of one launch, roughly: a conv's workgroups run in rounds of
+// one a CU, so a launch on part of the pixels takes as long as the rounds it
+// still needs (100 TFLOP/s over full rounds, as the larger layers run).
+static double launch_us(const k::ConvArgs& c, int tile) {
+    const double flops = 2.0 * c.N * c.Ho * c.Wo * c.Cout * c.K * c.groups;
+    const bool wino = k::is_wino_tile(tile);
+    const k::ConvTileShape sh = k::conv_tile_shape(tile);
+    const int64_t bn = wino ? (tile == k::kTileWino64 ? 64 : 32) : std::max(sh.bn, 1);
+    const int64_t pixels = static_cast<int64_t>(c.N) * c.Ho * c.Wo;
+    const int64_t bm = wino ? 128 : std::max(sh.bm, 1);
+    const int64_t wgs = (pixels + bm - 1) / bm * ((c.Cout + bn - 1) / bn) * c.groups * c.splits;
+    const double fill = static_cast<double>(wgs) / (256.0 * static_cast<double>((wgs + 255) / 256));
+    return 5.0 + flops / 1e8 / std::max(fill, 1e-3);
+}
+
+// The transfers of a sliced program are DMA copies on their own streams:
+// kernels that read or write host memory beside the steps' kernels hold those
+// up (a conv that takes 8 us alone took 41 beside a 41 us transfer kernel, on
+// 4 to 128 workgroups alike), the DMA engines do not.  With S slices the
+// upload, the steps and the download run side by side but for the first
+// slice's upload and the last one's rest, and each slice costs kSliceUs more
+// (copies wait for events, and events for copies, 15 to 35 us each); the
+// steps cost more too where a slice leaves the last round of workgroups
+// emptier.  S is the count up to kMaxIoSlices with the least estimate; the
+// estimate and the measured times agree on it for the sizes tried (us for S =
+// 1, 2, 3, 4; YOLOv8m C2f at 40x40, batch 16: 2148, 1659, 1388, 1524; its
+// SPPF: 692, 588, 654, 747; 64 -> 64 3x3 at 160x160: 287, 266, 262, 267;
+// 128 -> 64 1x1: 396, 369, 370, 386).
+// An unsliced program moves a tensor of up to kDirectBytes by the transfer
+// kernels themselves, on the session stream: they start and end with the
+// program's kernels, without a DMA copy's waits (96 -> 144 3x3 at 33x33: 62
+// -> 41 us).
+void Session::plan_io() {
+    constexpr double kSliceUs = 25.0, kLinkFloatsPerUs = 14000.0;  // 56 GB/s
+    constexpr int64_t kDirectBytes = 8 << 20;
+    constexpr int64_t kMaxIoSlices = 4;
+    Prepared& P = *prep_;
+    P.io.clear();
+    P.pull_relayout = P.push_relayout = P.pull_direct = P.push_direct = false;
+    const Plan& plan = P.plan;
+    if (!use_graph_ || concurrent_ || !P.segments.empty() || !P.in_chunks.empty()) return;
+    if (plan.input_bufs.size() != 1 || plan.outputs.size() != 1 || P.launches.empty()) return;
+    const int32_t in = plan.input_bufs[0], ob = plan.outputs[0].buf;
+    const size_t n = P.launches.size();
+
+    const Launch& f = P.launches.front();
+    if (f.kind == StepKind::Elt && f.elt == k::kEltCopy && n >= 2 && plan.steps.at(0).a.buf == in && dense4(f.a) &&
+        f.a.ptr == P.arena + plan.bufs.at(in).offset && same_dims(f.a, f.out) && rows4(f.out)) {
+        P.pull_relayout = true;
+        for (size_t i = 1; i < plan.steps.size(); ++i) {  // nothing else reads the planar input
+            const Step& s = plan.steps[i];
+            for (const VRef* v : {&s.a, &s.b, &s.c, &s.res, &s.cls_in})
+                if (v->buf == in) P.pull_relayout = false;
+        }
+    }
+    const Launch& l = P.launches.back();
+    const VRef& o = plan.outputs[0];
+    const size_t from = P.pull_relayout ? 1 : 0;
+    P.push_relayout = n > from + 1 && l.kind == StepKind::Elt && l.elt == k::kEltCopy &&
+                      plan.steps.back().out.buf == ob && plan.steps.back().a.buf != ob &&
+                      l.out.ptr == P.arena + plan.bufs.at(ob).offset + o.off && dense4(l.out) &&
+                      same_dims(l.a, l.out) && rows4(l.a) &&
+                      static_cast<int64_t>(P.outputs[0].nbytes) ==
+                          static_cast<int64_t>(sizeof(float)) * l.out.dims[0] * l.out.str[0];
+    if (P.push_relayout)
+        for (size_t i = 0; i + 1 < plan.steps.size(); ++i)
+            for (const VRef* v : {&plan.steps[i].out, &plan.steps[i].a, &plan.steps[i].b, &plan.steps[i].res})
+                if (v->buf == ob) P.push_relayout = false;  // only the copy touches the output
+    const size_t to = P.push_relayout ? n - 1 : n;
+
+    const int64_t N = plan.input_dims.at(0).empty() ? 0 : plan.input_dims[0][0];
+    int64_t in_floats = 1;
+    for (auto d : plan.input_dims[0]) in_floats *= d;
+    if (in_floats <= 0 || N <= 0) return;
+    const int64_t out_bytes = static_cast<int64_t>(P.outputs[0].nbytes);
+    const double up_us = static_cast<double>(in_floats) / kLinkFloatsPerUs;
+    const double down_us = static_cast<double>(out_bytes) / 4.0 / kLinkFloatsPerUs;
+    // the slice count by the estimate, `steps(S)` the steps' time in S slices
+    auto best_slices = [&](int64_t most, auto&& steps) {
+        if (io_slices_ > 0) return std::min<int64_t>(most, io_slices_);
+        int64_t best = 1;
+        double best_us = 0.0;
+        for (int64_t S = 1; S <= std::min(most, kMaxIoSlices); ++S) {
+            const double c = steps(S), part = static_cast<double>(S);
+            const double us = (up_us + c + down_us + (part - 1.0) * std::max({up_us, c, down_us})) / part + kSliceUs * part;
+            if (S == 1 || us < best_us) {
+                best = S;
+                best_us = us;
+            }
+        }
+        return best;
+    };
+    const bool both = P.pull_relayout && P.push_relayout && l.out.dims[0] == N;
+
+    // slices of the batch
+    if (both && N >= 2) {
+        bool ok = true;
+        auto batch_first = [&](const k::View& v) {
+            return v.ptr == nullptr || (v.rank >= 1 && v.dims[0] == N && v.str[0] > 0);
+        };
+        for (size_t i = from; i < to && ok; ++i) {
+            const Launch& b = P.launches[i];
+            if (b.kind == StepKind::ConvMfma)
+                ok = b.group.empty() && b.conv.N == N;
+            else if (b.kind == StepKind::ConvDirect)
+                ok = batch_first(b.direct.x) && batch_first(b.direct.y) && batch_first(b.direct.res);
+            else if (b.kind == StepKind::MaxPoolChain || b.kind == StepKind::MaxPool || b.kind == StepKind::Resize)
+                ok = batch_first(b.out) && batch_first(b.a) && batch_first(b.b) && batch_first(b.c);
+            else
+                ok = false;
+        }
+        const int64_t S = !ok ? 1 : best_slices(N, [&](int64_t n_slices) {
+            double us = 0.0;
+            for (size_t i = from; i < to; ++i) {
+                const Launch& b = P.launches[i];
+                if (b.kind != StepKind::ConvMfma) {
+                    us += 10.0 * static_cast<double>(n_slices);
+                    continue;
+                }
+                k::ConvArgs c = b.conv;
+                c.N = static_cast<int32_t>((N + n_slices - 1) / n_slices);
+                us += launch_us(c, b.tile) * static_cast<double>(n_slices);
+            }
+            return us;
+        });
+        ok = ok && S >= 2;
+        for (int64_t i = 0; ok && i < S; ++i) {
+            const int64_t n0 = N * i / S, m = N * (i + 1) / S - n0;
+            Prepared::IoSlice s;
+            s.pull = relayout_of(f.a, f.out, n0, m, 0, f.a.dims[2] * f.a.dims[3], true);
+            s.push = relayout_of(l.out, l.a, n0, m, 0, l.out.dims[2] * l.out.dims[3], false);
+            s.up.host = n0 * f.a.str[0];
+            s.up.width = m * f.a.str[0];
+            s.down.host = n0 * l.out.str[0];
+            s.down.width = m * l.out.str[0];
+            for (size_t j = from; j < to; ++j) {
+                Launch b = P.launches[j];
+                if (b.kind == StepKind::ConvMfma) {
+                    conv_slice(b.conv, n0, m);
+                } else if (b.kind == StepKind::ConvDirect) {
+                    b.direct.x = batch_slice(b.direct.x, N, n0, m);
+                    b.direct.y = batch_slice(b.direct.y, N, n0, m);
+                    b.direct.res = batch_slice(b.direct.res, N, n0, m);
+                } else {
+                    for (k::View* v : {&b.out, &b.a, &b.b, &b.c}) *v = batch_slice(*v, N, n0, m);
+                }
+                s.body.push_back(std::move(b));
+            }
+            P.io.push_back(std::move(s));
+        }
+        if (ok) return;
+        P.io.clear();
+    }
+
+    // slices of one image's output rows, each with the input rows it is the
+    // first to need (starting at even rows: a Winograd launch's 2x2 tiles
+    // stay those of the whole image, and so do the output's bits)
+    if (both && N == 1 && to - from == 1 && P.launches[from].kind == StepKind::ConvMfma) {
+        const Launch& b = P.launches[from];
+        const k::ConvArgs& c = b.conv;
+        const int64_t S = best_slices(static_cast<int64_t>(c.Ho) / 8, [&](int64_t n_slices) {
+            k::ConvArgs r = c;
+            r.Ho = static_cast<int32_t>((c.Ho + n_slices - 1) / n_slices);
+            return launch_us(r, b.tile) * static_cast<double>(n_slices);
+        });
+        if (b.group.empty() && c.splits == 1 && !c.up && !c.res && S >= 2) {
+            int64_t have = 0;  // input rows of the slices so far
+            for (int64_t i = 0; i < S; ++i) {
+                const int64_t r0 = c.Ho * i / S / 2 * 2, r1 = i + 1 < S ? c.Ho * (i + 1) / S / 2 * 2 : c.Ho;
+                int64_t need = (r1 - 1) * c.sh - c.ph + static_cast<int64_t>(c.KH - 1) * c.dh + 1;
+                need = i + 1 < S ? std::clamp<int64_t>(need, have, c.H) : c.H;
+                Prepared::IoSlice s;
+                s.pull = relayout_of(f.a, f.out, 0, 1, have * c.W, (need - have) * c.W, true);
+                s.push = relayout_of(l.out, l.a, 0, 1, r0 * c.Wo, (r1 - r0) * c.Wo, false);
+                s.up.host = have * c.W;
+                s.up.width = (need - have) * c.W;
+                s.up.pitch = f.a.str[1];
+                s.up.rows = f.a.dims[1];
+                s.down.host = r0 * c.Wo;
+                s.down.width = (r1 - r0) * c.Wo;
+                s.down.pitch = l.out.str[1];
+                s.down.rows = l.out.dims[1];
+                Launch r = b;
+                r.conv.row0 = static_cast<int32_t>(r0);
+                r.conv.Ho = static_cast<int32_t>(r1 - r0);
+                r.conv.y += r0 * c.y_sh;
+                s.body.push_back(std::move(r));
+                have = need;
+                P.io.push_back(std::move(s));
+            }
+            return;
+        }
+    }
+
+    Prepared::IoSlice s;
+    s.up.width = in_floats;
+    s.down.width = out_bytes / static_cast<int64_t>(sizeof(float));
+    if (P.pull_relayout) s.pull = relayout_of(f.a, f.out, 0, N, 0, f.a.dims[2] * f.a.dims[3], true);
+    if (P.push_relayout) s.push = relayout_of(l.out, l.a, 0, l.out.dims[0], 0, l.out.dims[2] * l.out.dims[3], false);
+    s.body.assign(P.launches.begin() + static_cast<int64_t>(from), P.launches.begin() + static_cast<int64_t>(to));
+    P.io.push_back(std::move(s));
+    P.pull_direct = 4 * in_floats <= kDirectBytes;
+    P.push_direct = P.push_relayout && out_bytes <= kDirectBytes;
+}
+
+// One run through the slices: uploads in order on copy_in_, each slice's
+// steps on the session stream once its upload has finished, its download on
+// copy_out_ once they have; a single slice stays on the session stream.
+void Session::run_io() {
+    Prepared& P = *prep_;
+    const Plan& plan = P.plan;
+    const HostTensor* t = inputs_[0];
+    float* staging = P.arena + plan.bufs.at(plan.input_bufs[0]).offset;
+    float* result = P.arena + plan.bufs.at(plan.outputs[0].buf).offset + plan.outputs[0].off;
+    const float* host = static_cast<const float*>(t->data);
+    const bool many = P.io.size() > 1;
+    // a kernel can read page-locked tensors only; the others go up by a copy
+    const bool direct = P.pull_direct && t->pinned && reinterpret_cast<uintptr_t>(host) % 16 == 0;
+    if (many && !copy_in_) PDEFA_HIP(hipStreamCreateWithFlags(&copy_in_, hipStreamNonBlocking));
+    if (many && !copy_out_) PDEFA_HIP(hipStreamCreateWithFlags(&copy_out_, hipStreamNonBlocking));
+    hipStream_t in = many ? copy_in_ : stream_, out = many ? copy_out_ : stream_;
+    auto copy = [](float* dst, const float* src, const Region& r, hipMemcpyKind kind, hipStream_t s) {
+        if (r.width <= 0) return;
+        const size_t width = sizeof(float) * static_cast<size_t>(r.width);
+        const size_t pitch = sizeof(float) * static_cast<size_t>(r.pitch);
+        if (r.rows <= 1)
+            PDEFA_HIP(hipMemcpyAsync(dst + r.host, src + r.host, width, kind, s));
+        else
+            PDEFA_HIP(hipMemcpy2DAsync(dst + r.host, pitch, src + r.host, pitch, width, static_cast<size_t>(r.rows),
+                                       kind, s));
+    };
+    auto upload = [&](Prepared::IoSlice& s) {
+        if (!direct)
+            copy(staging, host, s.up, hipMemcpyHostToDevice, in);
+        else
+            k::launch_copy_floats(staging, host, s.up.width, in);
+        if (many) {
+            if (!s.pulled) PDEFA_HIP(hipEventCreateWithFlags(&s.pulled, hipEventDisableTiming));
+            PDEFA_HIP(hipEventRecord(s.pulled, in));
+        }
+    };
+    // two uploads ahead of the steps: the host issues a slice's work while
+    // the next slices' copies run
+    size_t issued = 0;
+    for (size_t i = 0; i < P.io.size(); ++i) {
+        for (; issued < std::min(P.io.size(), i + 2); ++issued) upload(P.io[issued]);
+        Prepared::IoSlice& s = P.io[i];
+        if (many) PDEFA_HIP(hipStreamWaitEvent(stream_, s.pulled, 0));
+        if (P.pull_relayout && s.pull.P > 0) k::launch_planar_to_rows(s.pull, stream_);
+        if (s.body.size() > kGraphLaunches) {
+            if (!s.exec) capture_list(s.body, &s.graph, &s.exec);
+            PDEFA_HIP(hipGraphLaunch(s.exec, stream_));
+        } else {
+            for (const Launch& l : s.body) launch_one(l, stream_);
+        }
+        if (P.push_relayout) {
+            k::RelayoutArgs r = s.push;
+            if (P.push_direct) {
+                r.host = true;
+                r.mirror = r.dst;
+                r.dst = P.host_out[0];
+            }
+            k::launch_rows_to_planar(r, stream_);
+        }
+        if (many) {
+            if (!s.computed) PDEFA_HIP(hipEventCreateWithFlags(&s.computed, hipEventDisableTiming));
+            PDEFA_HIP(hipEventRecord(s.computed, stream_));
+            PDEFA_HIP(hipStreamWaitEvent(out, s.computed, 0));
+        }
+        if (!P.push_direct) copy(P.host_out[0], result, s.down, hipMemcpyDeviceToHost, out);
+    }
+    PDEFA_HIP(hipGetLastError());
+    if (many) PDEFA_HIP(hipStreamSynchronize(copy_in_));
+    PDEFA_HIP(hipStreamSynchronize(stream_));
+    if (many) PDEFA_HIP(hipStreamSynchronize(copy_out_));
+}
+
 void Session::upload_inputs() {
     const Plan& plan = prep_->plan;
     for (size_t i = 0; i < inputs_.size(); ++i) {
@@ -1355,7 +1685,8 @@ void Session::run() {
     if (!prep_ || prep_->plan.input_dims != dims) prepare(dims);
     const bool per_step = prof_fn_ != nullptr || std::getenv("ENGINE_PROFILE_CSV") != nullptr;
     const bool segmented = use_graph_ && !per_step && !prep_->segments.empty();
-    if (!segmented) upload_inputs();  // run_segments uploads (by slices) itself
+    const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged();
+    if (!segmented && !io) upload_inputs();  // run_segments uploads (by slices) itself
     if (per_step) {
         std::vector<double> ms;
         std::vector<std::string> labels;
@@ -1370,6 +1701,8 @@ void Session::run() {
         }
     } else if (segmented) {
         run_segments();
+    } else if (io) {
+        run_io();
     } else if (use_graph_) {
         if (!prep_->exec) {
             if (concurrent_) {
@@ -1393,7 +1726,7 @@ void Session::run() {
         launch_all(stream_);
         PDEFA_HIP(hipGetLastError());
     }
-    if (per_step || !use_graph_ || prep_->segments.empty()) {
+    if (!io && (per_step || !use_graph_ || prep_->segments.empty())) {
         download_outputs();
         PDEFA_HIP(hipStreamSynchronize(stream_));
     }

@@ -184,6 +184,23 @@ class Session {
         };
         std::vector<InChunk> in_chunks;
         size_t early_launches = 0;
+        // Programs between a layout copy of one input and one of one output
+        // (or either): the copies become transfers between the page-locked
+        // host tensors and the arena, and where the steps between them work
+        // image by image (or are one conv of one image), the batch (the
+        // output rows) is cut into slices whose transfers overlap the other
+        // slices' compute and each other.
+        struct IoSlice {
+            Region up, down;  // the slice of the input and of the output
+            k::RelayoutArgs pull, push;
+            std::vector<Launch> body;
+            hipGraph_t graph = nullptr;
+            hipGraphExec_t exec = nullptr;
+            hipEvent_t pulled = nullptr, computed = nullptr;
+        };
+        bool pull_relayout = false, push_relayout = false;
+        bool pull_direct = false, push_direct = false;  // transfers by kernels on the host memory
+        std::vector<IoSlice> io;  // empty: upload, program, download one after another
         ~Prepared();
     };
 
@@ -196,6 +213,8 @@ class Session {
     void plan_input_chunks();  // fills prep_->in_chunks (or leaves them empty)
     void plan_segments();  // fills prep_->segments (or leaves them empty)
     void run_segments();   // one run through the segments, downloads included
+    void plan_io();        // fills prep_->io (or leaves it empty)
+    void run_io();         // one run through the slices, transfers included
     void capture_concurrent();  // records the program as a multi-stream hipGraph
     void launch_one(const Launch& l, hipStream_t s);
     void upload_inputs();
@@ -238,6 +257,7 @@ class Session {
     hipStream_t copy_out_ = nullptr;         // downloads that overlap the program's later segments
     hipStream_t copy_in_ = nullptr;          // input slices uploaded while earlier chunks compute
     int input_chunks_ = 2;                   // PDEFA_INPUT_CHUNKS (<= 1: the input goes up whole)
+    int io_slices_ = 0;                      // PDEFA_IO_SLICES: at most this many slices (0: by size)
     int64_t early_hw_ = 80 * 80;             // PDEFA_EARLY_HW: smallest map the early steps produce
     bool concurrent_ = true;
     std::vector<const HostTensor*> inputs_;

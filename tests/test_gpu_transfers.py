@@ -1,0 +1,68 @@
+"""Programs whose edges are layout copies: the transfers by kernels and the
+sliced runs (PDEFA_IO_SLICES) give the bits of the same program run without
+either (PDEFA_HIP_GRAPH=0: upload, every step, download)."""
+import os
+
+import numpy as np
+import pytest
+
+from pdefa_amd import native, yolo_synth as ys
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(kind, c, h, w, batch):
+    if kind == "scdown":
+        return ys.build_scdown(c, c, h, n=batch, seed=3)[0]
+    b = ys.GraphBuilder()
+    y = ys._Yolo(b, np.random.default_rng(3), 0.0)
+    out = y.c2f(-1, c, c, 1, True, "block") if kind == "c2f" else y.sppf(-1, c, c, "block")
+    return b.model([batch, c, h, w], [batch, c, h, w], [out])
+
+
+def _run(path, xs, env, monkeypatch):
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    try:
+        eng = native.Engine(path)
+        try:
+            return [eng.run(x)[0].copy() for x in xs]
+        finally:
+            eng.close()
+    finally:
+        for k in env:
+            monkeypatch.delenv(k)
+
+
+def _check(model, shape, tmp_path, monkeypatch, slices):
+    path = os.path.join(tmp_path, "m.engine")
+    ys.save(model, path)
+    rng = np.random.default_rng(5)
+    xs = [rng.standard_normal(shape, dtype=np.float32) for _ in range(2)]
+    want = _run(path, xs, {"PDEFA_HIP_GRAPH": "0"}, monkeypatch)
+    assert not np.array_equal(want[0], want[1])
+    for s in slices:
+        print(f"[case] {shape} slices {s}", flush=True)
+        got = _run(path, xs + xs[:1], {"PDEFA_IO_SLICES": str(s)} if s else {}, monkeypatch)
+        for g, w in zip(got, want + want[:1]):
+            np.testing.assert_array_equal(g, w)
+
+
+# Output rows that do not divide by the slice count, odd widths (4-byte
+# accesses), one and two channels past a 64-wide tile, strides and kernel
+# sizes whose slices share input rows, tensors below and above the size from
+# which host tensors are page-locked.
+@pytest.mark.parametrize("cin,cout,k,s,hw", [
+    (64, 64, 3, 1, 40), (32, 66, 3, 1, 37), (16, 24, 3, 2, 65), (96, 144, 3, 2, 33), (64, 65, 1, 1, 50),
+    (128, 64, 1, 1, 31), (16, 16, 3, 1, 16), (24, 40, 3, 2, 18),
+])
+def test_single_conv_transfers(cin, cout, k, s, hw, tmp_path, monkeypatch):
+    model = ys.build_single_conv(cin, cout, k, s, hw, seed=3)[0]
+    _check(model, (1, cin, hw, hw), tmp_path, monkeypatch, [0, 1, 2, 3, 8])
+
+
+@pytest.mark.parametrize("kind,c,h,w,batch", [
+    ("c2f", 64, 20, 24, 5), ("c2f", 96, 13, 11, 2), ("sppf", 64, 21, 20, 3), ("scdown", 64, 22, 22, 4),
+])
+def test_block_transfers(kind, c, h, w, batch, tmp_path, monkeypatch):
+    _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8])
