@@ -494,7 +494,7 @@ PDEFA_EXPORT EngineStatus engine_run_simple(const char* model_path, const Engine
 
 namespace {
 
-using GemmFn = void (*)(const float*, const float*, float*, int64_t, int64_t, int64_t);
+using GemmFn = void (*)(const pdefa::MatmulHost&, int64_t, int64_t, int64_t);
 
 // The shape rules of ops::matmul (matmul.cpp:59-135): F32 only; rank > 2
 // on either side is batched [..., M, K] x [..., K, N] (or a 2-D B shared by
@@ -523,13 +523,13 @@ EngineStatus matmul_front(const EngineTensor* a, const EngineTensor* b, EngineTe
             const int64_t bstride = B.rank == 2 ? 0 : K * N;
             if (bstride && B.numel() < batch * K * N) return ENGINE_OK;
             for (int64_t i = 0; i < batch; ++i)
-                gemm(A.f32() + i * M * K, B.f32() + i * bstride, Cc.f32() + i * M * N, M, K, N);
+                gemm({A.f32() + i * M * K, B.f32() + i * bstride, Cc.f32() + i * M * N, A.pinned, B.pinned, Cc.pinned}, M, K, N);
             return ENGINE_OK;
         }
         if (A.rank != 2 || B.rank != 2 || Cc.rank != 2) return ENGINE_OK;
         const int64_t M = A.dims[0], K = A.dims[1], N = B.dims[1];
         if (B.dims[0] != K || Cc.dims[0] != M || Cc.dims[1] != N) return ENGINE_OK;
-        gemm(A.f32(), B.f32(), Cc.f32(), M, K, N);
+        gemm({A.f32(), B.f32(), Cc.f32(), A.pinned, B.pinned, Cc.pinned}, M, K, N);
         return ENGINE_OK;
     });
 }

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
 #include <vector>
 
 namespace pdefa {
@@ -316,9 +317,14 @@ struct RelayoutArgs {
 };
 void launch_planar_to_rows(const RelayoutArgs& a, hipStream_t s);
 void launch_rows_to_planar(const RelayoutArgs& a, hipStream_t s);
-// n contiguous floats between 16-byte aligned addresses, either of which may
-// be page-locked host memory.
-void launch_copy_floats(float* dst, const float* src, int64_t n, hipStream_t s);
+// Up to two runs of contiguous floats in one launch, between 16-byte aligned
+// addresses, either of which may be page-locked host memory.
+struct CopyRun {
+    float* dst = nullptr;
+    const float* src = nullptr;
+    int64_t n = 0;
+};
+void launch_copy_floats(std::initializer_list<CopyRun> runs, hipStream_t s);
 
 // Max pooling over logical [N, C, H, W] views (padding never wins).
 void launch_maxpool(const View& out, const View& in, int kh, int kw, int sh, int sw, int ph,
@@ -380,8 +386,9 @@ void launch_detect_decode(const DetectDecodeArgs& a, hipStream_t s);
 // Packs conv weights [Cout, Cin, KH, KW] (device, contiguous) into the packed
 // layout above.
 void launch_pack_conv_weights(float* dst, const float* w, int Cout, int Cin, int KH, int KW, hipStream_t s);
-// Packs a row-major B[K, N] matrix the same way (a 1x1 conv with Cin = K).
-void launch_pack_gemm_b(float* dst, const float* b, int K, int N, hipStream_t s);
+// Packs a row-major B[K, N] matrix the same way (a 1x1 conv with Cin = K) and
+// clears the N biases of that conv.
+void launch_pack_gemm_b(float* dst, const float* b, int K, int N, float* bias, hipStream_t s);
 
 // Elements of packed weights.
 int64_t packed_weight_elems(int Cout, int K);

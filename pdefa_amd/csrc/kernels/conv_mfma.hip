@@ -311,7 +311,10 @@ __global__ void pack_conv_weights_kernel(float* dst, const float* w, int Cout, i
     }
 }
 
-__global__ void pack_gemm_b_kernel(float* dst, const float* b, int K, int N, int ktiles, int64_t total) {
+__global__ void pack_gemm_b_kernel(float* dst, const float* b, int K, int N, int ktiles, int64_t total, float* bias) {
+    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < N;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+        bias[i] = 0.0f;
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
          i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const int kk = static_cast<int>(i % BK);
@@ -335,11 +338,11 @@ void launch_pack_conv_weights(float* dst, const float* w, int Cout, int Cin, int
                        total);
 }
 
-void launch_pack_gemm_b(float* dst, const float* b, int K, int N, hipStream_t s) {
+void launch_pack_gemm_b(float* dst, const float* b, int K, int N, float* bias, hipStream_t s) {
     const int ktiles = (K + BK - 1) / BK;
     const int64_t total = packed_weight_elems(N, K);
     const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 65535));
-    hipLaunchKernelGGL(pack_gemm_b_kernel, dim3(blocks), dim3(256), 0, s, dst, b, K, N, ktiles, total);
+    hipLaunchKernelGGL(pack_gemm_b_kernel, dim3(blocks), dim3(256), 0, s, dst, b, K, N, ktiles, total, bias);
 }
 
 }  // namespace k

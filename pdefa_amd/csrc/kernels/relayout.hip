@@ -183,12 +183,18 @@ void launch_relayout(const RelayoutArgs& a, hipStream_t s) {
     else go(relayout_kernel<IN, false, false>);
 }
 
-// n4 float4s and the tail floats after them, four loads in flight a lane.
-__global__ __launch_bounds__(kLanes) void copy_floats_kernel(float* dst, const float* src, int64_t n4, int tail) {
+// One run a blockIdx.y: its float4s, four loads in flight a lane, and the
+// floats after them.
+struct CopyRuns {
+    CopyRun r[2];
+};
+__global__ __launch_bounds__(kLanes) void copy_floats_kernel(CopyRuns runs) {
+    const CopyRun r = runs.r[blockIdx.y];
+    const int64_t n4 = r.n / 4;
     const int64_t tid = blockIdx.x * static_cast<int64_t>(kLanes) + threadIdx.x;
     const int64_t step = static_cast<int64_t>(gridDim.x) * kLanes;
-    const float4* s = reinterpret_cast<const float4*>(src);
-    float4* d = reinterpret_cast<float4*>(dst);
+    const float4* s = reinterpret_cast<const float4*>(r.src);
+    float4* d = reinterpret_cast<float4*>(r.dst);
     for (int64_t i = tid; i < n4; i += 4 * step) {
         float4 v[4];
 #pragma unroll
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(kLanes) void copy_floats_kernel(float* dst, const f
         for (int u = 0; u < 4; ++u)
             if (i + u * step < n4) d[i + u * step] = v[u];
     }
-    if (tid < tail) dst[4 * n4 + tid] = src[4 * n4 + tid];
+    if (tid < r.n - 4 * n4) r.dst[4 * n4 + tid] = r.src[4 * n4 + tid];
 }
 
 }  // namespace
@@ -205,13 +211,21 @@ __global__ __launch_bounds__(kLanes) void copy_floats_kernel(float* dst, const f
 void launch_planar_to_rows(const RelayoutArgs& a, hipStream_t s) { launch_relayout<true>(a, s); }
 void launch_rows_to_planar(const RelayoutArgs& a, hipStream_t s) { launch_relayout<false>(a, s); }
 
-void launch_copy_floats(float* dst, const float* src, int64_t n, hipStream_t s) {
-    if (n <= 0) return;
-    if (!dst || !src || !aligned16(dst) || !aligned16(src)) throw std::runtime_error("copy: pointers");
-    const int64_t n4 = n / 4;
-    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n4 + 4 * kLanes - 1) / (4 * kLanes), kTransferBlocks));
-    hipLaunchKernelGGL(copy_floats_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kLanes), 0, s, dst, src, n4,
-                       static_cast<int>(n % 4));
+void launch_copy_floats(std::initializer_list<CopyRun> runs, hipStream_t s) {
+    CopyRuns c;
+    unsigned count = 0;
+    int64_t most = 0;
+    for (const CopyRun& r : runs) {
+        if (r.n <= 0) continue;
+        if (count == 2 || !r.dst || !r.src || !aligned16(r.dst) || !aligned16(r.src))
+            throw std::runtime_error("copy: runs");
+        c.r[count++] = r;
+        most = std::max(most, r.n);
+    }
+    if (count == 0) return;
+    const int64_t per = 16 * kLanes;  // floats of a workgroup's loads in flight
+    const int64_t blocks = std::min<int64_t>((most + per - 1) / per, kTransferBlocks / count);
+    hipLaunchKernelGGL(copy_floats_kernel, dim3(static_cast<unsigned>(blocks), count), dim3(kLanes), 0, s, c);
 }
 
 }  // namespace k

@@ -1358,17 +1358,33 @@ static double launch_us(const k::ConvArgs& c, int tile) {
 // slice's upload and the last one's rest, and each slice costs kSliceUs more
 // (copies wait for events, and events for copies, 15 to 35 us each); the
 // steps cost more too where a slice leaves the last round of workgroups
-// emptier.  S is the count up to kMaxIoSlices with the least estimate; the
-// estimate and the measured times agree on it for the sizes tried (us for S =
-// 1, 2, 3, 4; YOLOv8m C2f at 40x40, batch 16: 2148, 1659, 1388, 1524; its
-// SPPF: 692, 588, 654, 747; 64 -> 64 3x3 at 160x160: 287, 266, 262, 267;
-// 128 -> 64 1x1: 396, 369, 370, 386).
+// emptier (steps(S): their time in S slices).  S is the count up to `most`
+// with the least estimate; it is the measured best for the sizes tried (us
+// for S = 1, 2, 3, 4; YOLOv8m C2f at 40x40, batch 16: 2148, 1659, 1388, 1524;
+// its SPPF: 692, 588, 654, 747; 64 -> 64 3x3 at 160x160: 287, 266, 262, 267;
+// 128 -> 64 1x1: 396, 369, 370, 386) or within 2% of it.
+static constexpr double kLinkFloatsPerUs = 14000.0;  // 56 GB/s
+template <typename F>
+static int64_t pipeline_slices(double up_us, double down_us, int64_t most, F&& steps) {
+    constexpr double kSliceUs = 25.0;
+    int64_t best = 1;
+    double best_us = 0.0;
+    for (int64_t S = 1; S <= most; ++S) {
+        const double c = steps(S), part = static_cast<double>(S);
+        const double us = (up_us + c + down_us + (part - 1.0) * std::max({up_us, c, down_us})) / part + kSliceUs * part;
+        if (S == 1 || us < best_us) {
+            best = S;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 // An unsliced program moves a tensor of up to kDirectBytes by the transfer
 // kernels themselves, on the session stream: they start and end with the
 // program's kernels, without a DMA copy's waits (96 -> 144 3x3 at 33x33: 62
 // -> 41 us).
 void Session::plan_io() {
-    constexpr double kSliceUs = 25.0, kLinkFloatsPerUs = 14000.0;  // 56 GB/s
     constexpr int64_t kDirectBytes = 8 << 20;
     constexpr int64_t kMaxIoSlices = 4;
     Prepared& P = *prep_;
@@ -1412,20 +1428,9 @@ void Session::plan_io() {
     const int64_t out_bytes = static_cast<int64_t>(P.outputs[0].nbytes);
     const double up_us = static_cast<double>(in_floats) / kLinkFloatsPerUs;
     const double down_us = static_cast<double>(out_bytes) / 4.0 / kLinkFloatsPerUs;
-    // the slice count by the estimate, `steps(S)` the steps' time in S slices
     auto best_slices = [&](int64_t most, auto&& steps) {
         if (io_slices_ > 0) return std::min<int64_t>(most, io_slices_);
-        int64_t best = 1;
-        double best_us = 0.0;
-        for (int64_t S = 1; S <= std::min(most, kMaxIoSlices); ++S) {
-            const double c = steps(S), part = static_cast<double>(S);
-            const double us = (up_us + c + down_us + (part - 1.0) * std::max({up_us, c, down_us})) / part + kSliceUs * part;
-            if (S == 1 || us < best_us) {
-                best = S;
-                best_us = us;
-            }
-        }
-        return best;
+        return pipeline_slices(up_us, down_us, std::min(most, kMaxIoSlices), steps);
     };
     const bool both = P.pull_relayout && P.push_relayout && l.out.dims[0] == N;
 
@@ -1570,7 +1575,7 @@ void Session::run_io() {
         if (!direct)
             copy(staging, host, s.up, hipMemcpyHostToDevice, in);
         else
-            k::launch_copy_floats(staging, host, s.up.width, in);
+            k::launch_copy_floats({{staging, host, s.up.width}}, in);
         if (many) {
             if (!s.pulled) PDEFA_HIP(hipEventCreateWithFlags(&s.pulled, hipEventDisableTiming));
             PDEFA_HIP(hipEventRecord(s.pulled, in));
@@ -1685,7 +1690,14 @@ void Session::run() {
     if (!prep_ || prep_->plan.input_dims != dims) prepare(dims);
     const bool per_step = prof_fn_ != nullptr || std::getenv("ENGINE_PROFILE_CSV") != nullptr;
     const bool segmented = use_graph_ && !per_step && !prep_->segments.empty();
-    const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged();
+    // (an input that lies in the memory of this run's output, the last run's
+    // output fed back, is read whole before any of the output is written)
+    auto in_output = [&] {
+        const char* a = static_cast<const char*>(inputs_[0]->data);
+        const char* h = reinterpret_cast<const char*>(prep_->host_out[0]);
+        return a < h + prep_->outputs[0].nbytes && h < a + inputs_[0]->nbytes;
+    };
+    const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged() && !in_output();
     if (!segmented && !io) upload_inputs();  // run_segments uploads (by slices) itself
     if (per_step) {
         std::vector<double> ms;
@@ -1883,14 +1895,23 @@ void Session::read_conv_input(const std::string& node, std::vector<float>& dst, 
 
 namespace {
 
+constexpr int kMatmulSlices = 4;  // most row slices of one product
+
 struct MatmulScratch {
     std::mutex mu;
     hipStream_t stream = nullptr;
+    hipStream_t up = nullptr, down = nullptr;  // a sliced product's transfers
+    hipEvent_t landed[kMatmulSlices] = {}, done[kMatmulSlices] = {};
     float* buf = nullptr;
     size_t cap = 0;  // floats
     ~MatmulScratch() {
         if (buf) (void)hipFree(buf);
-        if (stream) (void)hipStreamDestroy(stream);
+        for (hipEvent_t e : landed)
+            if (e) (void)hipEventDestroy(e);
+        for (hipEvent_t e : done)
+            if (e) (void)hipEventDestroy(e);
+        for (hipStream_t s : {stream, up, down})
+            if (s) (void)hipStreamDestroy(s);
     }
 };
 
@@ -1921,33 +1942,27 @@ MatmulLayout matmul_layout(int64_t M, int64_t K, int64_t N) {
     return L;
 }
 
-// Host A, B in; host C out; the device buffers at `base` (L.total() floats).
-void matmul_on(const MatmulLayout& L, float* base, const float* A, const float* B, float* C, int64_t M, int64_t K,
-               int64_t N, hipStream_t s) {
+// Rows [r0, r0 + rows) of the product, from A and the packed B at `base`.
+void matmul_rows(const MatmulLayout& L, float* base, int64_t r0, int64_t rows, int64_t K, int64_t N, hipStream_t s) {
     float* dA = base;
-    float* dB = dA + L.nA;
-    float* dP = dB + L.nB;
+    float* dP = dA + L.nA + L.nB;
     float* dBias = dP + L.nP;
     float* dC = dBias + L.nBias;
     float* dW = dC + L.nC;
-    PDEFA_HIP(hipMemcpyAsync(dA, A, sizeof(float) * M * K, hipMemcpyHostToDevice, s));
-    PDEFA_HIP(hipMemcpyAsync(dB, B, sizeof(float) * K * N, hipMemcpyHostToDevice, s));
-    PDEFA_HIP(hipMemsetAsync(dBias, 0, L.nBias * sizeof(float), s));
-    k::launch_pack_gemm_b(dP, dB, static_cast<int>(K), static_cast<int>(N), s);
     k::ConvArgs c;
-    c.x = dA;
+    c.x = dA + r0 * K;
     c.N = 1;
-    c.H = static_cast<int32_t>(M);
+    c.H = static_cast<int32_t>(rows);
     c.W = 1;
     c.Cin = static_cast<int32_t>(K);
-    c.x_sn = M * K;
+    c.x_sn = rows * K;
     c.x_sh = K;
     c.x_sw = K;
-    c.y = dC;
-    c.Ho = static_cast<int32_t>(M);
+    c.y = dC + r0 * N;
+    c.Ho = static_cast<int32_t>(rows);
     c.Wo = 1;
     c.Cout = static_cast<int32_t>(N);
-    c.y_sn = M * N;
+    c.y_sn = rows * N;
     c.y_sh = N;
     c.y_sw = N;
     c.wpk = dP;
@@ -1958,14 +1973,81 @@ void matmul_on(const MatmulLayout& L, float* base, const float* A, const float* 
     c.kt_per_split = L.ls.kt_per_split;
     c.ws = L.ls.splits > 1 ? dW : nullptr;
     k::launch_conv_mfma(c, L.ls.tile, K % 4 == 0, s);
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// Host A, B in; host C out; the device buffers at `base` (L.total() floats).
+// Up to kKernelBytes a page-locked operand moves by a kernel of the stream
+// (kernels/relayout.hip), larger ones by DMA copies.
+void matmul_on(const MatmulLayout& L, float* base, const MatmulHost& h, int64_t M, int64_t K, int64_t N,
+               hipStream_t s) {
+    constexpr int64_t kKernelBytes = 8 << 20;
+    float* dA = base;
+    float* dB = dA + L.nA;
+    float* dP = dB + L.nB;
+    float* dBias = dP + L.nP;
+    float* dC = dBias + L.nBias;
+    auto move = [&](float* dst, const float* src, int64_t n, bool pinned, hipMemcpyKind kind) {
+        const int64_t bytes = static_cast<int64_t>(sizeof(float)) * n;
+        if (pinned && bytes <= kKernelBytes && aligned16(src) && aligned16(dst))
+            k::launch_copy_floats({{dst, src, n}}, s);
+        else
+            PDEFA_HIP(hipMemcpyAsync(dst, src, static_cast<size_t>(bytes), kind, s));
+    };
+    if (h.a_pinned && h.b_pinned && 4 * M * K <= kKernelBytes && 4 * K * N <= kKernelBytes && aligned16(h.A) &&
+        aligned16(h.B)) {
+        k::launch_copy_floats({{dA, h.A, M * K}, {dB, h.B, K * N}}, s);
+    } else {
+        move(dA, h.A, M * K, h.a_pinned, hipMemcpyHostToDevice);
+        move(dB, h.B, K * N, h.b_pinned, hipMemcpyHostToDevice);
+    }
+    k::launch_pack_gemm_b(dP, dB, static_cast<int>(K), static_cast<int>(N), dBias, s);
+    matmul_rows(L, base, 0, M, K, N, s);
     PDEFA_HIP(hipGetLastError());
-    PDEFA_HIP(hipMemcpyAsync(C, dC, sizeof(float) * M * N, hipMemcpyDeviceToHost, s));
+    move(h.C, dC, M * N, h.c_pinned, hipMemcpyDeviceToHost);
     PDEFA_HIP(hipStreamSynchronize(s));
+}
+
+// The same in `slices` row slices: B goes up first, then A slice by slice on
+// the upload stream while earlier slices multiply and theirs of C go down
+// (3001 x 2047 by 2047 x 1733: 1405 us whole, 1093, 1033 and 1031 in 2, 3 and
+// 4 slices; each of C's elements is summed as in the whole product).
+void matmul_sliced(const MatmulLayout& L, MatmulScratch& sc, const MatmulHost& h, int64_t M, int64_t K, int64_t N,
+                   int64_t slices) {
+    float* dA = sc.buf;
+    float* dB = dA + L.nA;
+    float* dP = dB + L.nB;
+    float* dBias = dP + L.nP;
+    float* dC = dBias + L.nBias;
+    for (hipStream_t* s : {&sc.up, &sc.down})
+        if (!*s) PDEFA_HIP(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
+    for (int64_t i = 0; i < slices; ++i)
+        for (hipEvent_t* e : {&sc.landed[i], &sc.done[i]})
+            if (!*e) PDEFA_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    PDEFA_HIP(hipMemcpyAsync(dB, h.B, sizeof(float) * K * N, hipMemcpyHostToDevice, sc.stream));
+    k::launch_pack_gemm_b(dP, dB, static_cast<int>(K), static_cast<int>(N), dBias, sc.stream);
+    auto row = [&](int64_t i) { return M * i / slices; };
+    for (int64_t i = 0; i < slices; ++i) {
+        const int64_t r0 = row(i), rows = row(i + 1) - r0;
+        PDEFA_HIP(hipMemcpyAsync(dA + r0 * K, h.A + r0 * K, sizeof(float) * rows * K, hipMemcpyHostToDevice, sc.up));
+        PDEFA_HIP(hipEventRecord(sc.landed[i], sc.up));
+    }
+    for (int64_t i = 0; i < slices; ++i) {
+        const int64_t r0 = row(i), rows = row(i + 1) - r0;
+        PDEFA_HIP(hipStreamWaitEvent(sc.stream, sc.landed[i], 0));
+        matmul_rows(L, sc.buf, r0, rows, K, N, sc.stream);
+        PDEFA_HIP(hipGetLastError());
+        PDEFA_HIP(hipEventRecord(sc.done[i], sc.stream));
+        PDEFA_HIP(hipStreamWaitEvent(sc.down, sc.done[i], 0));
+        PDEFA_HIP(hipMemcpyAsync(h.C + r0 * N, dC + r0 * N, sizeof(float) * rows * N, hipMemcpyDeviceToHost, sc.down));
+    }
+    for (hipStream_t s : {sc.up, sc.stream, sc.down}) PDEFA_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace
 
-void device_matmul(const float* A, const float* B, float* C, int64_t M, int64_t K, int64_t N) {
+void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {
     if (!device_available()) throw std::runtime_error("no HIP device available for ops_matmul");
     if (M <= 0 || K <= 0 || N <= 0) return;
     const MatmulLayout L = matmul_layout(M, K, N);
@@ -1979,10 +2061,29 @@ void device_matmul(const float* A, const float* B, float* C, int64_t M, int64_t 
         PDEFA_HIP(hipMalloc(&sc.buf, L.total() * sizeof(float)));
         sc.cap = L.total();
     }
-    matmul_on(L, sc.buf, A, B, C, M, K, N, sc.stream);
+    // slices need page-locked operands, and a C apart from A (a slice of C
+    // goes down while later slices of A go up)
+    int64_t slices = 1;
+    const bool apart = h.C + M * N <= h.A || h.A + M * K <= h.C;
+    if (h.a_pinned && h.b_pinned && h.c_pinned && apart)
+        slices = pipeline_slices(static_cast<double>(M * K) / kLinkFloatsPerUs,
+                                 static_cast<double>(M * N) / kLinkFloatsPerUs,
+                                 std::min<int64_t>(kMatmulSlices, M / 256), [&](int64_t n) {
+                                     k::ConvArgs c;
+                                     c.N = c.Wo = c.groups = 1;
+                                     c.Ho = static_cast<int32_t>((M + n - 1) / n);
+                                     c.Cout = static_cast<int32_t>(N);
+                                     c.K = static_cast<int32_t>(K);
+                                     c.splits = L.ls.splits;
+                                     return launch_us(c, L.ls.tile) * static_cast<double>(n);
+                                 });
+    if (slices > 1)
+        matmul_sliced(L, sc, h, M, K, N, slices);
+    else
+        matmul_on(L, sc.buf, h, M, K, N, sc.stream);
 }
 
-void device_matmul_noalloc(const float* A, const float* B, float* C, int64_t M, int64_t K, int64_t N) {
+void device_matmul_noalloc(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {
     if (!device_available()) throw std::runtime_error("no HIP device available for ops_matmul");
     if (M <= 0 || K <= 0 || N <= 0) return;
     const MatmulLayout L = matmul_layout(M, K, N);
@@ -1998,7 +2099,7 @@ void device_matmul_noalloc(const float* A, const float* B, float* C, int64_t M, 
         throw std::invalid_argument(os.str());
     }
     // the null stream: nothing is created
-    matmul_on(L, base, A, B, C, M, K, N, nullptr);
+    matmul_on(L, base, h, M, K, N, nullptr);
 }
 
 }  // namespace pdefa

@@ -66,3 +66,37 @@ def test_single_conv_transfers(cin, cout, k, s, hw, tmp_path, monkeypatch):
 ])
 def test_block_transfers(kind, c, h, w, batch, tmp_path, monkeypatch):
     _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8])
+
+
+# Row counts around the slice rule's smallest slice, a remainder row per slice,
+# K % 4 != 0 (4-byte operand loads), products below and above the sizes from
+# which operands are page-locked and sliced, and C in A's memory (never sliced).
+@pytest.mark.parametrize("m,k,n", [(1, 5, 7), (300, 260, 300), (512, 512, 512), (2049, 1023, 1030), (3001, 2047, 601)])
+def test_matmul_transfers(m, k, n):
+    from pdefa_amd import pdefa as api
+
+    print(f"[case] matmul {m}x{k}x{n}", flush=True)
+    rng = np.random.default_rng(7)
+    for _ in range(2):
+        a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+        ta, tb = (api.Tensor(native.tensor_from_numpy(v)) for v in (a, b))
+        out = api.empty(m, n)
+        api.ops_matmul(ta, tb, out)
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        # k products of unit variance, each partial sum rounded to 2^-24 of
+        # itself: an error of about sqrt(k) * sqrt(k) * 2^-24 at the most
+        np.testing.assert_allclose(out.numpy(), want, rtol=0, atol=k * 2.0**-24 * 4 + 1e-6)
+
+
+def test_matmul_into_its_own_operand():
+    from pdefa_amd import pdefa as api
+
+    print("[case] matmul 1024 into A", flush=True)
+    rng = np.random.default_rng(8)
+    a, b = (rng.standard_normal((1024, 1024), dtype=np.float32) for _ in range(2))
+    ta, tb = (api.Tensor(native.tensor_from_numpy(v)) for v in (a, b))
+    apart = api.empty(1024, 1024)
+    api.ops_matmul(ta, tb, apart)
+    api.ops_matmul(ta, tb, ta)
+    np.testing.assert_allclose(ta.numpy(), apart.numpy(), rtol=0, atol=1024 * 2.0**-24 * 4)
+    np.testing.assert_array_equal(tb.numpy(), b)
