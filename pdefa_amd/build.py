@@ -26,6 +26,7 @@ SOURCES = [
     "kernels/conv_mfma_tiles_c.hip",
     "kernels/conv_mfma_tiles_d.hip",
     "kernels/conv_mfma_tiles_e.hip",
+    "kernels/conv_mfma_tiles_split.hip",
     "kernels/conv_wino.hip",
     "kernels/conv_wino_strip.hip",
     "kernels/ops.hip",

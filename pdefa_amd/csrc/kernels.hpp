@@ -86,11 +86,17 @@ enum ConvTile : int32_t {
     kTile32x16K4 = 18,     // 1 wave tile of 32x16, K split in 4
     kTile16x32K8W8 = 19,   // 1 wave tile of 16x32, K split in 8
     kTile32x16K8W8 = 20,   // 1 wave tile of 32x16, K split in 8
-    kNumConvShapes = 21,   // tile ids (implicit-GEMM and Winograd)
+    // The implicit GEMM on the bf16 matrix cores with each f32 operand split
+    // into three bf16 terms (conv_mfma_tile.hpp); finite weights only
+    kTileSplit128x128W8 = 21,  // 2x4 waves of 64x32
+    kNumConvShapes = 22,   // tile ids (implicit-GEMM, Winograd and split)
 };
+inline bool is_split_tile(int tile) { return tile == kTileSplit128x128W8; }
 inline bool is_wino_tile(int tile) { return tile == kTileWino64 || tile == kTileWino32; }
-// An implicit-GEMM tile id (conv_mfma_kernel).
-inline bool is_gemm_tile(int tile) { return tile >= 0 && tile < kNumConvShapes && !is_wino_tile(tile); }
+// An f32 implicit-GEMM tile id (conv_mfma_kernel).
+inline bool is_gemm_tile(int tile) {
+    return tile >= 0 && tile < kNumConvShapes && !is_wino_tile(tile) && !is_split_tile(tile);
+}
 ConvTileShape conv_tile_shape(int tile);
 const char* conv_tile_name(int tile);
 

@@ -19,6 +19,7 @@ bool launch_conv_tiles_d(int tile, const ConvArgs& a, bool vec, dim3 grid, hipSt
 bool launch_group_tiles_d(int tile, const ConvGroupArgs& g, hipStream_t s);
 bool launch_conv_tiles_e(int tile, const ConvArgs& a, bool vec, dim3 grid, hipStream_t s);
 bool launch_group_tiles_e(int tile, const ConvGroupArgs& g, hipStream_t s);
+bool launch_conv_tiles_split(int tile, const ConvArgs& a, bool vec, dim3 grid, hipStream_t s);
 
 // Sums split-K partials in split order, then bias + activation + residual.
 // Every lane of a workgroup runs the same number of iterations (a lane past
@@ -87,18 +88,19 @@ constexpr ConvTileShape kShapes[kNumConvShapes] = {
     {128, 64, 32, 32, 1},  {64, 64, 32, 32, 2},  {128, 128, 64, 32, 1}, {64, 128, 32, 32, 1},
     {32, 64, 32, 32, 4},   {32, 32, 32, 32, 8},  {0, 0, 0, 0, 0},       {0, 0, 0, 0, 0},
     {16, 16, 16, 16, 4},   {16, 32, 16, 32, 4},  {32, 16, 32, 16, 4},   {16, 32, 16, 32, 8},
-    {32, 16, 32, 16, 8},
+    {32, 16, 32, 16, 8},   {128, 128, 64, 32, 1},
 };
 constexpr const char* kNames[kNumConvShapes] = {
     "128x128",  "128x64",    "64x128",    "64x64",     "128x32",    "64x32k2",   "32x64k2",
     "32x32k4",  "128x64w8",  "64x64k2w8", "128x128w8", "64x128w8",  "32x64k4w8", "32x32k8w8",
-    "wino64",   "wino32",    "16x16k4",   "16x32k4",   "32x16k4",   "16x32k8w8", "32x16k8w8"};
+    "wino64",   "wino32",    "16x16k4",   "16x32k4",   "32x16k4",   "16x32k8w8", "32x16k8w8",
+    "split128x128w8"};
 
 }  // namespace
 
 
 ConvTileShape conv_tile_shape(int tile) {
-    if (!is_gemm_tile(tile)) return {0, 0, 0, 0, 0};
+    if (!is_gemm_tile(tile) && !is_split_tile(tile)) return {0, 0, 0, 0, 0};
     return kShapes[tile];
 }
 const char* conv_tile_name(int tile) { return tile >= 0 && tile < kNumConvShapes ? kNames[tile] : "?"; }
@@ -123,11 +125,11 @@ double conv_cost(int64_t M, int Cout, int ktiles, int t, int splits, int steps) 
     constexpr double kKernelCycles = 10000.0;  // launch + completion of one kernel
     constexpr double kWgCycles = 1500.0;       // workgroup start-up (first loads)
     constexpr double kStepFloor = 2200.0;      // latency floor of one pipeline step
-    constexpr double kEff[kNumConvShapes] = {1.0, 0.8, 0.8, 0.85, 0.8, 0.75, 0.75, 0.7, 0.85, 0.85, 0.9,
+    constexpr double kEff[kTileSplit128x128W8] = {1.0, 0.8, 0.8, 0.85, 0.8, 0.75, 0.75, 0.7, 0.85, 0.85, 0.9,
                                              0.85, 0.75, 0.65, 1.0, 1.0, 0.55, 0.6, 0.6, 0.55, 0.55};
     // 8-wave tiles hide part of a step's latency behind the other wave of the
     // SIMD; a 16x16 block's step runs a quarter of the MFMA chain
-    constexpr double kFloorScale[kNumConvShapes] = {1,    1,    1,    1,   1,   1,   1,   1,   0.75, 0.75, 0.75,
+    constexpr double kFloorScale[kTileSplit128x128W8] = {1,    1,    1,    1,   1,   1,   1,   1,   0.75, 0.75, 0.75,
                                                     0.75, 0.75, 0.8,  1,   1,   0.6, 0.7, 0.7, 0.55, 0.55};
     const ConvTileShape& sh = kShapes[t];
     const int64_t wgs0 = ((M + sh.bm - 1) / sh.bm) * ((Cout + sh.bn - 1) / sh.bn);
@@ -249,7 +251,7 @@ void launch_conv_mfma(const ConvArgs& a, int tile, bool vec, hipStream_t s) {
     b.fd_splits = make_fastdiv(a.splits);
     if (!(launch_conv_tiles_a(tile, b, vec, grid, s) || launch_conv_tiles_b(tile, b, vec, grid, s) ||
           launch_conv_tiles_c(tile, b, vec, grid, s) || launch_conv_tiles_d(tile, b, vec, grid, s) ||
-          launch_conv_tiles_e(tile, b, vec, grid, s)))
+          launch_conv_tiles_e(tile, b, vec, grid, s) || launch_conv_tiles_split(tile, b, vec, grid, s)))
         fail("unknown tile");
     if (a.splits > 1) {
         const int64_t total = M * a.Cout * a.groups;
@@ -260,7 +262,7 @@ void launch_conv_mfma(const ConvArgs& a, int tile, bool vec, hipStream_t s) {
 
 void launch_conv_mfma_group(const ConvArgs* probs, int count, int tile, hipStream_t s) {
     const ConvTileShape sh = conv_tile_shape(tile);
-    if (sh.bm == 0) fail("unknown tile");
+    if (sh.bm == 0 || is_split_tile(tile)) fail("unknown tile");
     if (count < 1 || count > kMaxConvGroup) fail("group size out of range");
     ConvGroupArgs g;
     g.count = count;

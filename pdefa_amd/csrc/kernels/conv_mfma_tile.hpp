@@ -59,23 +59,27 @@ namespace k {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 namespace {
 
 constexpr int BK = kConvBK;         // 32: K per slice and per packed block
 constexpr int LDS_STRIDE = BK + 4;  // floats; 16-byte aligned rows, conflict-free float4 reads
+// Row of a split stage, in 4-byte words: three bf16 planes of BK, padded so
+// that the 16-byte reads of 8 consecutive rows fall on distinct banks
+constexpr int SPLIT_STRIDE = 3 * BK / 2 + 4;
 constexpr int kXcds = 8;
 
 // Stage buffers (two stages of KG A and B slices), then the per-row output
 // offset table of the epilogue (three int64 per tile row: output, residual,
 // upsampled output).
-template <int BM, int BN, int KG>
+template <int BM, int BN, int KG, bool SPLIT = false>
 constexpr size_t lds_stage_bytes() {
-    return sizeof(float) * 2 * KG * (BM + BN) * LDS_STRIDE;
+    return sizeof(float) * 2 * KG * (BM + BN) * (SPLIT ? SPLIT_STRIDE : LDS_STRIDE);
 }
-template <int BM, int BN, int KG>
+template <int BM, int BN, int KG, bool SPLIT = false>
 constexpr size_t lds_bytes() {
-    return lds_stage_bytes<BM, BN, KG>() + 3 * sizeof(int64_t) * BM;
+    return lds_stage_bytes<BM, BN, KG, SPLIT>() + 3 * sizeof(int64_t) * BM;
 }
 
 }  // namespace
@@ -139,8 +143,32 @@ __device__ __forceinline__ int xcd_tile(int lin, int total) {
 // pass and an upsampled copy (the launchers check).
 constexpr int kEpiPlain = 0, kEpiFix = 1, kEpiUp = 2, kEpiFixOnly = 3;
 
+// x as three bf16 terms whose sum is x: each takes the leading 8 significand
+// bits of what the ones before it leave, by truncation, so every difference
+// is exact and 24 bits are covered; a term is the upper half of its float.
+// A NaN stays one in the terms.  INF: x may be infinite, and goes to the last
+// term alone then, which meets only the leading term of the other operand:
+// the products with it are those of x itself (beside a finite x's other terms
+// an infinite leading one would meet zeros).
+struct SplitTerms {
+    uint32_t t[3];
+};
+template <bool INF>
+__device__ __forceinline__ SplitTerms split_terms(float x) {
+    const bool fin = !INF || __builtin_fabsf(x) < __builtin_inff();
+    const float v = fin ? x : 0.0f;
+    SplitTerms s;
+    s.t[0] = __float_as_uint(v) & 0xffff0000u;
+    const float r = v - __uint_as_float(s.t[0]);
+    s.t[1] = __float_as_uint(r) & 0xffff0000u;
+    const float l = r - __uint_as_float(s.t[1]);
+    s.t[2] = __float_as_uint(fin ? l : x);
+    return s;
+}
+
 // One BM x BN output tile (m block bx, n block by) of K split bz of problem a.
-template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI>
+// SPLIT: the products on the bf16 matrix cores (see split_terms).
+template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI, bool SPLIT = false>
 __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const int by, const int bz,
                                           const int grp) {
     constexpr int WAVES_M = BM / WM;
@@ -171,8 +199,10 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
 
     extern __shared__ __attribute__((aligned(16))) float smem[];
     // stage st, slice g: A tile at smem + (st*KG + g)*BM*LDS_STRIDE, B tiles after all A tiles
-    auto As = [&](int st, int g) { return smem + (st * KG + g) * BM * LDS_STRIDE; };
-    auto Bs = [&](int st, int g) { return smem + 2 * KG * BM * LDS_STRIDE + (st * KG + g) * BN * LDS_STRIDE; };
+    constexpr int STRIDE = SPLIT ? SPLIT_STRIDE : LDS_STRIDE;
+    static_assert(!SPLIT || (KG == 1 && MB == 32 && VEC), "split tiles");
+    auto As = [&](int st, int g) { return smem + (st * KG + g) * BM * STRIDE; };
+    auto Bs = [&](int st, int g) { return smem + 2 * KG * BM * STRIDE + (st * KG + g) * BN * STRIDE; };
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -321,9 +351,28 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
         for (int i = 0; i < B_ROWS; ++i)
             br[i] = *reinterpret_cast<const floatx4*>(brow[i] + static_cast<int64_t>(kb) * (kConvBN * BK));
     };
+    // the three planes of a float4 chunk of a split row (weights are finite:
+    // the planner checks)
+    auto store_split = [&](auto inf_c, float* row, floatx4 v) {
+        SplitTerms t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = split_terms<decltype(inf_c)::value>(v[e]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p)  // the upper halves of two words as one
+            *reinterpret_cast<uint2*>(row + p * (BK / 2) + cc * 2) =
+                make_uint2(__builtin_amdgcn_perm(t[1].t[p], t[0].t[p], 0x07060302u),
+                           __builtin_amdgcn_perm(t[3].t[p], t[2].t[p], 0x07060302u));
+    };
     auto store_step = [&](int st, const floatx4* ar, const floatx4* br) {
         float* A = As(st, cg);
         float* B = Bs(st, cg);
+        if constexpr (SPLIT) {
+#pragma unroll
+            for (int r = 0; r < A_ROWS; ++r) store_split(std::true_type{}, &A[(r0 + ROW_STEP * r) * STRIDE], ar[r]);
+#pragma unroll
+            for (int i = 0; i < B_ROWS; ++i) store_split(std::false_type{}, &B[(r0 + ROW_STEP * i) * STRIDE], br[i]);
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < A_ROWS; ++r)
             *reinterpret_cast<floatx4*>(&A[(r0 + ROW_STEP * r) * LDS_STRIDE + cc * 4]) = ar[r];
@@ -333,18 +382,89 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     };
 
     AccT acc[TM][TN];
+    // split tiles: the leading products and the small ones are summed apart,
+    // so that the small ones do not add their roundings to the large sum
+    AccT low[SPLIT ? TM : 1][SPLIT ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int e = 0; e < NE; ++e) acc[i][j][e] = 0.0f;
+            for (int e = 0; e < NE; ++e) {
+                acc[i][j][e] = 0.0f;
+                if constexpr (SPLIT) low[i][j][e] = 0.0f;
+            }
 
     // 32x32 blocks: lane (half h, row l % 32) reads k = 8q + 4h .. +3 and feeds
     // them to MFMA steps (q, 0..3) of 2 k each; 16x16 blocks: lane (quarter h,
     // row l % 16) reads k = 16q + 4h .. +3 for steps (q, 0..3) of 4 k each.
     constexpr int KQ = MB == 32 ? 8 : 16;  // k per quad of MFMA steps
     const int krd = MB == 32 ? half * 4 : (lane >> 4) * 4;
+    // Split step: the products of LDS stage st, and between them the split and
+    // the LDS stores of the next step's loads (next: into stage st ^ 1, which
+    // no wave reads before the barrier), so that the vector ALU works through
+    // the splits while the matrix core multiplies.  Both 16-wide quarters'
+    // fragments are read ahead of their products.
+    // v_mfma_f32_32x32x16_bf16: lane half h supplies k = 16q + 8h .. +7 of its
+    // row.  The six products of terms down to 2^-16 of the leading one; the
+    // dropped ones are below 2^-23 of it.
+    //
+    // What bounds it: per 32-wide step of a 128 x 128 tile a SIMD has 1536
+    // cycles of MFMAs, about 1250 of vector ALU (5.5 to 8.5 instructions a
+    // loaded element) and the CU 1400 of LDS traffic, which overlap only in
+    // part (about 3800 measured).  16 x 40x40 images, us against the f32 tile
+    // of the launch-shape table: 768 -> 384 1x1 114 / 161 (198 TFLOP/s), 384
+    // -> 384 1x1 67 / 88; 16 x 20x20, 1152 -> 576: 62 / 97.  Tried: four
+    // waves of 64x64 (140) and 128 x 64 tiles, two workgroups a CU (124);
+    // one quarter's fragments at a time (129); the groups of products held in
+    // order by scheduling barriers (122); a wave-uniform branch around the
+    // handling of infinities (219: it spills).
+    auto split_step = [&](int st, const floatx4* ar, const floatx4* br, bool next) {
+        if constexpr (SPLIT) {
+            constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+            constexpr int CHUNKS = A_ROWS + B_ROWS, KQS = BK / 16, GROUPS = 6 * KQS, FQ = KQS;
+            const float* Ab = As(st, 0);
+            const float* Bb = Bs(st, 0);
+            float* An = As(st ^ 1, 0);
+            float* Bn = Bs(st ^ 1, 0);
+            bf16x8 av[FQ][TM][3], bv[FQ][TN][3];
+            auto frags = [&](int q) {
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+#pragma unroll
+                    for (int tm = 0; tm < TM; ++tm)
+                        av[q % FQ][tm][p] = *reinterpret_cast<const bf16x8*>(
+                            &Ab[(wave_m * WM + tm * MB + lcol) * STRIDE + p * (BK / 2) + q * 8 + half * 4]);
+#pragma unroll
+                    for (int tn = 0; tn < TN; ++tn)
+                        bv[q % FQ][tn][p] = *reinterpret_cast<const bf16x8*>(
+                            &Bb[(wave_n * WN + tn * MB + lcol) * STRIDE + p * (BK / 2) + q * 8 + half * 4]);
+                }
+            };
+#pragma unroll
+            for (int q = 0; q + 1 < FQ; ++q) frags(q);
+            static_for<GROUPS>([&](auto gc) {
+                constexpr int G = decltype(gc)::value, q = G / 6, P = G % 6;
+                if (P == 0 && q + FQ - 1 < KQS) frags(q + FQ - 1);
+#pragma unroll
+                for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+                    for (int tn = 0; tn < TN; ++tn) {
+                        AccT& c = P == 5 ? acc[tm][tn] : low[tm][tn];
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[q % FQ][tm][PA[P]], bv[q % FQ][tn][PB[P]], c, 0, 0,
+                                                                    0);
+                    }
+                if (next)
+#pragma unroll
+                    for (int i = CHUNKS * G / GROUPS; i < CHUNKS * (G + 1) / GROUPS; ++i) {
+                        if (i < A_ROWS)
+                            store_split(std::true_type{}, &An[(r0 + ROW_STEP * i) * STRIDE], ar[i]);
+                        else
+                            store_split(std::false_type{}, &Bn[(r0 + ROW_STEP * (i - A_ROWS)) * STRIDE], br[i - A_ROWS]);
+                    }
+            });
+        }
+    };
     auto compute_step = [&](int st) {
         const float* Ab = As(st, wg);
         const float* Bb = Bs(st, wg);
@@ -391,7 +511,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     // this split's partial slab) and in the residual; -1 past the last row.
     // Built while the first steps' loads are in flight, read after the
     // pipeline's barriers.
-    int64_t* s_yoff = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(smem) + lds_stage_bytes<BM, BN, KG>());
+    int64_t* s_yoff = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(smem) + lds_stage_bytes<BM, BN, KG, SPLIT>());
     int64_t* s_roff = s_yoff + BM;
     int64_t* s_uoff = s_roff + BM;
     if (tid < BM) {
@@ -441,6 +561,12 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
         constexpr int R = J % PF;  // register stage of step it
         constexpr int L = J % 2;   // LDS stage of step it
         if (load) load_step(kb_begin + (it + PF) * KG, areg[R], breg[R]);
+        if constexpr (SPLIT) {
+            constexpr int S = (R + 1) % PF;
+            split_step(L, areg[S], breg[S], store);
+            stage_sync();
+            return;
+        }
         compute_step(L);
         if (store) store_step(L ^ 1, areg[(R + 1) % PF], breg[(R + 1) % PF]);
         stage_sync();
@@ -452,6 +578,15 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
         constexpr int J = decltype(jc)::value;
         if (it + J < nk) iteration(it + J, jc, it + J + PF < nk, it + J + 1 < nk);
     });
+
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < NE; ++e) acc[i][j][e] += low[i][j][e];
+    }
 
     // ---- output.  The row table was written before the prologue barrier
     // (every split has at least one step, checked by the launcher).  A tile
@@ -690,7 +825,7 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
 // One problem; grid (m tiles, n tiles, K splits), tiles in XCD order with the
 // m tile fastest (neighbouring output rows share input rows, all tiles of one
 // n block share weights).
-template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI>
+template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI, bool SPLIT = false>
 __global__ __launch_bounds__((tile_threads<BM, BN, WM, WN, KG>())) void conv_mfma_kernel(ConvArgs a) {
     const int gx = gridDim.x, gxy = gridDim.x * gridDim.y;
     const int tile_id = xcd_tile(blockIdx.x + gx * blockIdx.y + gxy * blockIdx.z, gxy * gridDim.z);
@@ -698,7 +833,7 @@ __global__ __launch_bounds__((tile_threads<BM, BN, WM, WN, KG>())) void conv_mfm
     const int bxy = tile_id - bz * gxy;
     const int by = fdiv(bxy, a.fd_gx);
     const int grp = fdiv(bz, a.fd_splits);
-    conv_tile<BM, BN, WM, WN, KG, PF, VEC, EPI>(a, bxy - by * gx, by, bz - grp * a.splits, grp);
+    conv_tile<BM, BN, WM, WN, KG, PF, VEC, EPI, SPLIT>(a, bxy - by * gx, by, bz - grp * a.splits, grp);
 }
 
 // Several independent problems in one launch (no split-K): a 1-D grid over
@@ -716,19 +851,19 @@ __global__ __launch_bounds__((tile_threads<BM, BN, WM, WN, KG>())) void conv_mfm
 
 namespace {
 
-template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI>
+template <int BM, int BN, int WM, int WN, int KG, int PF, bool VEC, int EPI, bool SPLIT = false>
 void launch_one(const ConvArgs& a, dim3 grid, hipStream_t s) {
-    constexpr size_t bytes = lds_bytes<BM, BN, KG>();
-    static_assert(lds_stage_bytes<BM, BN, KG>() >= sizeof(float) * KG * BM * BN,
+    constexpr size_t bytes = lds_bytes<BM, BN, KG, SPLIT>();
+    static_assert(SPLIT || lds_stage_bytes<BM, BN, KG>() >= sizeof(float) * KG * BM * BN,
                   "slice reduction fits in the stage buffers");
     static std::once_flag once;
     std::call_once(once, [] {
         if (bytes > 65536)
             (void)hipFuncSetAttribute(
-                reinterpret_cast<const void*>(&conv_mfma_kernel<BM, BN, WM, WN, KG, PF, VEC, EPI>),
+                reinterpret_cast<const void*>(&conv_mfma_kernel<BM, BN, WM, WN, KG, PF, VEC, EPI, SPLIT>),
                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
     });
-    hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WM, WN, KG, PF, VEC, EPI>), grid,
+    hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WM, WN, KG, PF, VEC, EPI, SPLIT>), grid,
                        dim3(tile_threads<BM, BN, WM, WN, KG>()), bytes, s, a);
 }
 
@@ -793,6 +928,17 @@ void launch_tile(const ConvArgs& a, bool vec, dim3 grid, hipStream_t s) {
     } else {
         launch_one<BM, BN, WM, WN, KG, kPrefetch, false, kEpiPlain>(a, grid, s);
     }
+}
+
+template <int BM, int BN, int WM, int WN>
+void launch_split_tile(const ConvArgs& a, dim3 grid, hipStream_t s) {
+    const int epi = epi_of(a);
+    if (epi == kEpiUp)
+        launch_one<BM, BN, WM, WN, 1, kPrefetch, true, kEpiUp, true>(a, grid, s);
+    else if (epi == kEpiFix)
+        launch_one<BM, BN, WM, WN, 1, kPrefetch, true, kEpiFixOnly, true>(a, grid, s);
+    else
+        launch_one<BM, BN, WM, WN, 1, kPrefetch, true, kEpiPlain, true>(a, grid, s);
 }
 
 }  // namespace

@@ -386,6 +386,7 @@ class Planner {
         fuse_steps();
         split_decode();
         group_convs();
+        split_long_gemms();
         allocate();
         check_bounds();
         return std::move(plan_);
@@ -1075,7 +1076,7 @@ class Planner {
             }
             if (k::is_wino_tile(opt_.force_tile)) {
                 if (wino) ls = {opt_.force_tile, 1, static_cast<int>((K + k::kConvBK - 1) / k::kConvBK)};
-            } else if (k::is_gemm_tile(opt_.force_tile)) {
+            } else if (k::is_gemm_tile(opt_.force_tile) || (k::is_split_tile(opt_.force_tile) && s.vec && G == 1 && finite_weight(n.inputs[1]))) {
                 const int kg = k::conv_tile_shape(opt_.force_tile).kg;
                 const int steps_total = static_cast<int>((K + k::kConvBK - 1) / k::kConvBK + kg - 1) / kg;
                 const int want = std::max(1, std::min(opt_.force_splits, steps_total));
@@ -1352,7 +1353,7 @@ class Planner {
             // a conv whose output feeds a nearest 2x Resize right after it also
             // writes the upsampled copy (the FPN's upsample into its concat)
             // (not a compat-SiLU conv: its float64 second pass rewrites only y)
-            if (st[i].kind == StepKind::ConvMfma && st[i].vec && !k::is_wino_tile(st[i].tile) && i + 1 < st.size() &&
+            if (st[i].kind == StepKind::ConvMfma && st[i].vec && k::is_gemm_tile(st[i].tile) && i + 1 < st.size() &&
                 st[i].act != k::kActSiluWinogradForm && st[i + 1].kind == StepKind::Resize &&
                 views_equal(st[i + 1].a, st[i].out)) {
                 const VRef& y = st[i].out;
@@ -1645,6 +1646,47 @@ class Planner {
             for (const VRef& v : wr) check(v, static_cast<int64_t>(i), "write");
         }
         for (const VRef& v : plan_.outputs) check(v, -1, "graph output");
+    }
+
+    // Every value of constant r (a conv's weight) is finite: the split tile
+    // handles infinite inputs only.
+    bool finite_weight(int32_t r) const {
+        const HostTensor& w = m_.weights.at(static_cast<size_t>(-1000 - r));
+        if (w.dtype != kF32) return false;
+        const uint32_t* v = static_cast<const uint32_t*>(w.data);
+        const int64_t n = w.numel();
+        uint32_t bad = 0;
+        for (int64_t i = 0; i < n; ++i) bad |= (v[i] & 0x7f800000u) == 0x7f800000u;
+        return bad == 0;
+    }
+
+    // Long implicit GEMMs to the split tile (PlanOptions::split_terms): those
+    // whose output channels fill its 128-wide columns to 90%, whose tiles
+    // fill half the CUs and whose K is at least 768.  Measured on YOLOv8m's
+    // layers at batch 16 (us, the launch-shape table's f32 tile / split):
+    // with Cout 384 and 576, K from 384 to 3456 79 / 62 to 236 / 157 (1.28 to
+    // 1.51 times faster); with Cout 192 (75% of the columns) 1.04 to 1.12
+    // times faster at K 384 to 1728 and slower at 192, with Cout 96 1.07 at
+    // K 192 and slower at 96, with Cout 64 slower; 3x3 stride-1 layers
+    // stay with Winograd, 114 against 165.  The wide layers with K below 768
+    // are the entry convs of C2f blocks: their rounding decides which side of
+    // a SiLU jump some outputs of the 3x3 layers behind them take, and the 20
+    // us each would save are not worth moving those.
+    void split_long_gemms() {
+        if (!opt_.split_terms) return;
+        for (Step& s : plan_.steps) {
+            if (s.kind != StepKind::ConvMfma || !k::is_gemm_tile(s.tile) || s.group >= 0 || s.groups != 1 || !s.vec)
+                continue;
+            const int64_t M = s.out.dims[0] * s.out.dims[2] * s.out.dims[3], cout = s.out.dims[1];
+            const int64_t K = s.a.dims[1] * s.KH * s.KW;
+            const int64_t cols = (cout + 127) / 128;
+            if (K < 768 || (M + 127) / 128 * cols < 128 || 10 * cout < 9 * 128 * cols) continue;
+            if (!finite_weight(m_.nodes[s.node].inputs[1])) continue;
+            s.tile = k::kTileSplit128x128W8;
+            s.splits = 1;
+            s.kt_per_split = static_cast<int32_t>((K + k::kConvBK - 1) / k::kConvBK);
+            s.ws_buf = -1;
+        }
     }
 
     // Length of the leading run of steps that process each image on its own

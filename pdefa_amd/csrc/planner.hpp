@@ -141,6 +141,9 @@ struct PlanOptions {
     // > 0: Plan::early_steps covers the leading per-image steps whose outputs
     // have at least this many pixels (H * W)
     int64_t early_hw = 0;
+    // Long implicit GEMMs run on the bf16 matrix cores, each f32 operand as
+    // three bf16 terms (k::kTileSplit128x128W8).
+    bool split_terms = false;
     // The program's first layout copy (of an input) and last one (of an
     // output) may run as transfers that overlap other steps: the memory they
     // touch is shared with nothing.

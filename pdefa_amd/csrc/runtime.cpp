@@ -682,6 +682,8 @@ void Session::prepare(const std::vector<std::vector<int64_t>>& dims) {
                         ? early_hw_
                         : 0;
     opts.pin_io = use_graph_ && !concurrent_;
+    // PDEFA_SPLIT_TERMS=0: every conv on the f32 matrix cores
+    opts.split_terms = opts.force_tile < 0 && env_flag("PDEFA_SPLIT_TERMS", true);
     if (autotune_) {
         opts.tune_conv = [this](const ConvQuery& q) { return tune_conv(q, stream_); };
         // grouped launches change the program order; the concurrent capture
