@@ -431,6 +431,7 @@ Session::~Session() {
         release_prepared();
     } catch (...) {
     }
+    if (stream_) (void)hipStreamSynchronize(stream_);  // images of a set_images that no run followed
     for (hipStream_t s : side_streams_) (void)hipStreamDestroy(s);
     if (copy_out_) (void)hipStreamDestroy(copy_out_);
     if (copy_in_) (void)hipStreamDestroy(copy_in_);
@@ -558,8 +559,9 @@ std::vector<LetterboxGeometry> Session::set_images(int32_t idx, const std::vecto
         total += static_cast<size_t>(im.width) * im.height * im.channels;
         total = (total + 255) / 256 * 256;
     }
-    // the previous run's upload has finished reading the pinned staging
-    if (stream_) PDEFA_HIP(hipStreamSynchronize(stream_));
+    if (!stream_) PDEFA_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    // the previous images' upload has finished reading the pinned staging
+    PDEFA_HIP(hipStreamSynchronize(stream_));
     if (staged_.size() < inputs_.size()) staged_.resize(inputs_.size());
     StagedInput& st = staged_[idx];
     st.images.clear();
@@ -570,6 +572,13 @@ std::vector<LetterboxGeometry> Session::set_images(int32_t idx, const std::vecto
         PDEFA_HIP(hipHostMalloc(reinterpret_cast<void**>(&st.host_px), total, hipHostMallocDefault));
         st.host_cap = total;
     }
+    if (total > st.dev_cap) {
+        if (st.dev_px) (void)hipFree(st.dev_px);
+        st.dev_px = nullptr;
+        st.dev_cap = 0;
+        PDEFA_HIP(hipMalloc(reinterpret_cast<void**>(&st.dev_px), total));
+        st.dev_cap = total;
+    }
     st.tw = tw;
     st.th = th;
     st.scale = scale;
@@ -578,7 +587,9 @@ std::vector<LetterboxGeometry> Session::set_images(int32_t idx, const std::vecto
     size_t off = 0;
     for (const ImageRef& im : images) {
         const size_t n = static_cast<size_t>(im.width) * im.height * im.channels;
+        // each image goes up while the next one is copied to the staging
         std::memcpy(st.host_px + off, im.pixels, n);
+        PDEFA_HIP(hipMemcpyAsync(st.dev_px + off, st.host_px + off, n, hipMemcpyHostToDevice, stream_));
         StagedImage si;
         si.offset = off;
         si.img = im;
@@ -604,6 +615,8 @@ Session::Prepared::~Prepared() {
         if (c.graph) (void)hipGraphDestroy(c.graph);
         if (c.ready) (void)hipEventDestroy(c.ready);
     }
+    if (early_exec) (void)hipGraphExecDestroy(early_exec);
+    if (early_graph) (void)hipGraphDestroy(early_graph);
     for (Segment& g : segments) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -1242,10 +1255,11 @@ void Session::run_segments() {
     const Plan& plan = P.plan;
     if (!copy_out_) PDEFA_HIP(hipStreamCreateWithFlags(&copy_out_, hipStreamNonBlocking));
     if (P.in_chunks.empty() || has_staged()) {
+        // nothing to overlap: the early launches on the whole batch
         upload_inputs();
-        for (Prepared::InChunk& c : P.in_chunks) {
-            if (!c.exec) capture_list(c.launches, &c.graph, &c.exec);
-            PDEFA_HIP(hipGraphLaunch(c.exec, stream_));
+        if (P.early_launches > 0) {
+            if (!P.early_exec) capture_launches(0, P.early_launches - 1, &P.early_graph, &P.early_exec);
+            PDEFA_HIP(hipGraphLaunch(P.early_exec, stream_));
         }
     } else {
         if (!copy_in_) PDEFA_HIP(hipStreamCreateWithFlags(&copy_in_, hipStreamNonBlocking));
@@ -1625,17 +1639,6 @@ void Session::upload_inputs() {
         float* dst = prep_->arena + plan.bufs.at(plan.input_bufs[i]).offset;
         if (i < staged_.size() && !staged_[i].images.empty()) {
             StagedInput& st = staged_[i];
-            const StagedImage& last = st.images.back();
-            const size_t bytes = last.offset + static_cast<size_t>(last.img.width) * last.img.height * last.img.channels;
-            if (bytes > st.dev_cap) {
-                PDEFA_HIP(hipStreamSynchronize(stream_));
-                if (st.dev_px) (void)hipFree(st.dev_px);
-                st.dev_px = nullptr;
-                st.dev_cap = 0;
-                PDEFA_HIP(hipMalloc(reinterpret_cast<void**>(&st.dev_px), bytes));
-                st.dev_cap = bytes;
-            }
-            PDEFA_HIP(hipMemcpyAsync(st.dev_px, st.host_px, bytes, hipMemcpyHostToDevice, stream_));
             const size_t plane = static_cast<size_t>(st.tw) * st.th;
             for (size_t b = 0; b < st.images.size(); ++b) {
                 const StagedImage& si = st.images[b];
@@ -2100,8 +2103,9 @@ void device_matmul_noalloc(const MatmulHost& h, int64_t M, int64_t K, int64_t N)
            << " bytes of the static scratch array";
         throw std::invalid_argument(os.str());
     }
-    // the null stream: nothing is created
-    matmul_on(L, base, h, M, K, N, nullptr);
+    // the null stream: nothing is created; DMA copies: a first launch of the
+    // transfer kernels would load their code object into device memory
+    matmul_on(L, base, {h.A, h.B, h.C, false, false, false}, M, K, N, nullptr);
 }
 
 }  // namespace pdefa

@@ -76,8 +76,8 @@ class Session {
     // Input `idx` becomes the letterbox of `images` (batch = images.size(),
     // planar fp32 [n, 3, th, tw]) computed on the device at the next run: the
     // 8-bit pixels are copied now into pinned staging memory (the caller may
-    // release them), uploaded and letterboxed on the session stream before
-    // the program.  Returns each image's geometry.  set_input(idx, ...)
+    // release them) and their upload starts; they are letterboxed on the
+    // session stream before the program.  Returns each image's geometry.  set_input(idx, ...)
     // replaces it.
     std::vector<LetterboxGeometry> set_images(int32_t idx, const std::vector<ImageRef>& images, int32_t tw,
                                               int32_t th, float scale, float pad);
@@ -184,6 +184,8 @@ class Session {
         };
         std::vector<InChunk> in_chunks;
         size_t early_launches = 0;
+        hipGraph_t early_graph = nullptr;  // the early launches on the whole batch
+        hipGraphExec_t early_exec = nullptr;
         // Programs between a layout copy of one input and one of one output
         // (or either): the copies become transfers between the page-locked
         // host tensors and the arena, and where the steps between them work

@@ -1,6 +1,8 @@
 """Programs whose edges are layout copies: the transfers by kernels and the
 sliced runs (PDEFA_IO_SLICES) give the bits of the same program run without
-either (PDEFA_HIP_GRAPH=0: upload, every step, download)."""
+either (PDEFA_HIP_GRAPH=0: upload, every step, download).  The products here
+grow ops_matmul's scratch, so this file runs after test_zz_no_alloc, which
+watches it grow."""
 import os
 
 import numpy as np
@@ -100,3 +102,43 @@ def test_matmul_into_its_own_operand():
     api.ops_matmul(ta, tb, ta)
     np.testing.assert_allclose(ta.numpy(), apart.numpy(), rtol=0, atol=1024 * 2.0**-24 * 4)
     np.testing.assert_array_equal(tb.numpy(), b)
+
+
+def test_images_twice_before_a_run_and_one_after(tmp_path, monkeypatch):
+    """Images go up while set_images copies them: a second set_images before
+    the run replaces the first one's, a larger one grows the staging, and a
+    run after them reads the last."""
+    from pdefa_amd import pdefa as api
+
+    print("[case] images staged twice", flush=True)
+    path = os.path.join(tmp_path, "n.engine")
+    ys.save(ys.build_yolov8("n", seed=0, imgsz=(96, 160)), path)
+    rng = np.random.default_rng(6)
+    small = [rng.integers(0, 256, (90, 150, 3), dtype=np.uint8) for _ in range(4)]
+    large = [rng.integers(0, 256, (480, 333, 3), dtype=np.uint8) for _ in range(4)]
+
+    def session():
+        ctx = api.Context()
+        return api.Session(ctx, api.Model(ctx, path))
+
+    def stage(sess, images):
+        sess.set_images(0, [api.Image.from_array(i) for i in images], 160, 96, 1.0 / 255.0, 114.0 / 255.0)
+
+    def out(sess):
+        sess.run()
+        return sess.output(0).numpy().copy()
+
+    want = []
+    for images in (small, large):
+        sess = session()
+        stage(sess, images)
+        want.append(out(sess))
+    assert not np.array_equal(*want)
+    sess = session()
+    for images in (small, large):
+        stage(sess, images)
+    np.testing.assert_array_equal(out(sess), want[1])
+    np.testing.assert_array_equal(out(sess), want[1])
+    stage(sess, small)
+    np.testing.assert_array_equal(out(sess), want[0])
+    stage(sess, large)  # and no run
