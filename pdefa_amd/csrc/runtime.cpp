@@ -1763,11 +1763,11 @@ void Session::run() {
 double Session::replay(int32_t iters) {
     if (!prep_ || runs == 0) throw std::runtime_error("replay needs a completed run");
     hipEvent_t a, b;
+    if (use_graph_ && !concurrent_ && !prep_->exec)
+        capture_launches(0, prep_->launches.size() - 1, &prep_->graph, &prep_->exec);
     PDEFA_HIP(hipEventCreate(&a));
     PDEFA_HIP(hipEventCreate(&b));
     PDEFA_HIP(hipEventRecord(a, stream_));
-    if (use_graph_ && !concurrent_ && !prep_->exec)
-        capture_launches(0, prep_->launches.size() - 1, &prep_->graph, &prep_->exec);
     for (int32_t i = 0; i < iters; ++i) {
         if (prep_->exec)
             PDEFA_HIP(hipGraphLaunch(prep_->exec, stream_));
