@@ -1399,7 +1399,7 @@ static int64_t pipeline_slices(double up_us, double down_us, int64_t most, F&& s
 // An unsliced program moves a tensor of up to kDirectBytes by the transfer
 // kernels themselves, on the session stream: they start and end with the
 // program's kernels, without a DMA copy's waits (96 -> 144 3x3 at 33x33: 62
-// -> 41 us).
+// -> 41 us; a pass of YOLOv8n b1, whose head is 2.8 MB: 561 -> 558).
 void Session::plan_io() {
     constexpr int64_t kDirectBytes = 8 << 20;
     constexpr int64_t kMaxIoSlices = 4;
@@ -1558,7 +1558,8 @@ void Session::plan_io() {
     s.body.assign(P.launches.begin() + static_cast<int64_t>(from), P.launches.begin() + static_cast<int64_t>(to));
     P.io.push_back(std::move(s));
     P.pull_direct = 4 * in_floats <= kDirectBytes;
-    P.push_direct = P.push_relayout && out_bytes <= kDirectBytes;
+    // (the offset of a buffer in the arena is a multiple of 256 bytes)
+    P.push_direct = out_bytes <= kDirectBytes && (P.push_relayout || o.off % 4 == 0);
 }
 
 // One run through the slices: uploads in order on copy_in_, each slice's
@@ -1613,7 +1614,7 @@ void Session::run_io() {
         }
         if (P.push_relayout) {
             k::RelayoutArgs r = s.push;
-            if (P.push_direct) {
+            if (P.push_direct) {  // straight to the host
                 r.host = true;
                 r.mirror = r.dst;
                 r.dst = P.host_out[0];
@@ -1625,7 +1626,10 @@ void Session::run_io() {
             PDEFA_HIP(hipEventRecord(s.computed, stream_));
             PDEFA_HIP(hipStreamWaitEvent(out, s.computed, 0));
         }
-        if (!P.push_direct) copy(P.host_out[0], result, s.down, hipMemcpyDeviceToHost, out);
+        if (P.push_direct && !P.push_relayout)
+            k::launch_copy_floats({{P.host_out[0], result, s.down.width}}, stream_);
+        else if (!P.push_direct)
+            copy(P.host_out[0], result, s.down, hipMemcpyDeviceToHost, out);
     }
     PDEFA_HIP(hipGetLastError());
     if (many) PDEFA_HIP(hipStreamSynchronize(copy_in_));
