@@ -1963,6 +1963,79 @@ Schedule schedule_plan(const Plan& p, int max_streams) {
     return sc;
 }
 
+namespace {
+
+// A dense row-major rank-4 [N, C, H, W] view.
+bool dense4(const VRef& v) {
+    return v.rank == 4 && v.str[3] == 1 && v.str[2] == v.dims[3] && v.str[1] == v.dims[2] * v.dims[3] &&
+           v.str[0] == v.dims[1] * v.str[1];
+}
+// A channels-last one whose pixels follow each other evenly.
+bool rows4(const VRef& v) {
+    return v.rank == 4 && v.str[1] == 1 && v.str[3] >= v.dims[1] && v.str[2] == v.dims[3] * v.str[3] && v.str[0] >= 0;
+}
+
+}  // namespace
+
+IoShape io_shape(const Plan& p) {
+    IoShape io;
+    if (p.input_bufs.size() != 1 || p.outputs.size() != 1 || p.input_dims.at(0).empty() || p.steps.size() < 2) return io;
+    const int32_t in = p.input_bufs[0], ob = p.outputs[0].buf;
+    const int64_t N = p.input_dims[0][0];
+    const Step& f = p.steps.front();
+    const Step& l = p.steps.back();
+    io.pull = f.kind == StepKind::Elt && f.elt == k::kEltCopy && f.a.buf == in && f.a.off == 0 && dense4(f.a) &&
+              dims_of(f.a) == dims_of(f.out) && rows4(f.out);
+    std::vector<VRef> rd, wr;
+    for (size_t i = 1; i < p.steps.size(); ++i) {  // nothing else reads the planar input
+        step_views(p.steps[i], rd, wr);
+        for (const VRef& v : rd)
+            if (v.buf == in) io.pull = false;
+    }
+    const size_t from = io.pull ? 1 : 0;
+    int64_t out_elems = 1;
+    for (auto d : p.output_dims.at(0)) out_elems *= d;
+    io.push = p.steps.size() > from + 1 && l.kind == StepKind::Elt && l.elt == k::kEltCopy && l.out.buf == ob &&
+              l.a.buf != ob && l.out.off == p.outputs[0].off && dense4(l.out) && dims_of(l.a) == dims_of(l.out) &&
+              rows4(l.a) && out_elems == l.out.dims[0] * l.out.str[0];
+    for (size_t i = 0; i + 1 < p.steps.size(); ++i) {  // only the copy touches the output
+        step_views(p.steps[i], rd, wr);
+        for (const auto* vs : {&rd, &wr})
+            for (const VRef& v : *vs)
+                if (v.buf == ob) io.push = false;
+    }
+    if (!io.pull || !io.push || l.out.dims[0] != N) return io;
+    const size_t to = p.steps.size() - 1;
+
+    if (N >= 2) {
+        auto batch_first = [&](const VRef& v) {
+            return v.buf == -1 || (v.rank >= 1 && v.dims[0] == N && v.str[0] > 0);
+        };
+        for (size_t i = from; i < to; ++i) {
+            const Step& s = p.steps[i];
+            bool ok = false;
+            if (s.kind == StepKind::ConvMfma)
+                ok = s.group < 0 && s.a.dims[0] == N;
+            else if (s.kind == StepKind::ConvDirect)
+                ok = batch_first(s.a) && batch_first(s.out) && (!s.has_res || batch_first(s.res));
+            else if (s.kind == StepKind::MaxPool || s.kind == StepKind::Resize)
+                ok = batch_first(s.a) && batch_first(s.out);
+            else if (s.kind == StepKind::MaxPoolChain)
+                ok = batch_first(s.a) && batch_first(s.out) && batch_first(s.b) && batch_first(s.c);
+            if (!ok) return io;
+        }
+        io.slices = IoSlices::Batch;
+    } else if (N == 1 && to - from == 1) {
+        // the conv's rows are the copies' rows: it reads the whole of what the
+        // first one wrote, and the last one reads the whole of what it writes
+        const Step& s = p.steps[from];
+        if (s.kind == StepKind::ConvMfma && s.group < 0 && s.splits == 1 && !s.has_res && s.up.buf == -1 &&
+            views_equal(s.a, f.out) && views_equal(l.a, s.out))
+            io.slices = IoSlices::Rows;
+    }
+    return io;
+}
+
 Plan build_plan(const Model& m, const std::vector<std::vector<int64_t>>& input_dims, const PlanOptions& opt) {
     Planner p(m, input_dims, opt);
     return p.run();
@@ -2003,6 +2076,9 @@ std::string describe_plan(const Model& m, const Plan& p) {
     os << "arena";  // element offset of every buffer
     for (size_t b = 0; b < p.bufs.size(); ++b) os << " b" << b << "@" << p.bufs[b].offset;
     os << "\n";
+    const IoShape io = io_shape(p);
+    os << "transfers pull=" << io.pull << " push=" << io.push << " slices="
+       << (io.slices == IoSlices::Batch ? "batch" : io.slices == IoSlices::Rows ? "rows" : "none") << "\n";
     return os.str();
 }
 

@@ -166,6 +166,19 @@ struct Schedule {
 };
 Schedule schedule_plan(const Plan& p, int max_streams);
 
+// Which of a program's edges may run as transfers between the page-locked
+// host tensors and the arena, and in what slices the steps between them may
+// run, so that a slice's transfers overlap the others' steps.
+enum class IoSlices : int32_t { None, Batch, Rows };
+struct IoShape {
+    bool pull = false;  // the first step is a planar input's copy to channels-last
+    bool push = false;  // the last one is a channels-last tensor's copy to the planar output
+    // Batch: the images; Rows: the output rows of the one conv of one image
+    // that lies between the copies
+    IoSlices slices = IoSlices::None;
+};
+IoShape io_shape(const Plan& p);
+
 // Human-readable dump (one line per step) for tests and debugging.
 std::string describe_plan(const Model& m, const Plan& p);
 

@@ -1315,22 +1315,6 @@ void Session::run_segments() {
 
 namespace {
 
-// A dense row-major rank-4 [N, C, H, W] view.
-bool dense4(const k::View& v) {
-    return v.rank == 4 && v.str[3] == 1 && v.str[2] == v.dims[3] && v.str[1] == v.dims[2] * v.dims[3] &&
-           v.str[0] == v.dims[1] * v.str[1];
-}
-// A channels-last one whose pixels follow each other evenly.
-bool rows4(const k::View& v) {
-    return v.rank == 4 && v.str[1] == 1 && v.str[3] >= v.dims[1] && v.str[2] == v.dims[3] * v.str[3] && v.str[0] >= 0;
-}
-bool same_dims(const k::View& a, const k::View& b) {
-    if (a.rank != b.rank) return false;
-    for (int d = 0; d < a.rank; ++d)
-        if (a.dims[d] != b.dims[d]) return false;
-    return true;
-}
-
 // Pixels [p0, p0 + P) of images [n0, n0 + N) of a planar/channels-last pair.
 k::RelayoutArgs relayout_of(const k::View& planar, const k::View& rows, int64_t n0, int64_t N, int64_t p0, int64_t P,
                             bool to_rows) {
@@ -1409,33 +1393,14 @@ void Session::plan_io() {
     const Plan& plan = P.plan;
     if (!use_graph_ || concurrent_ || !P.segments.empty() || !P.in_chunks.empty()) return;
     if (plan.input_bufs.size() != 1 || plan.outputs.size() != 1 || P.launches.empty()) return;
-    const int32_t in = plan.input_bufs[0], ob = plan.outputs[0].buf;
+    const IoShape io = io_shape(plan);
+    P.pull_relayout = io.pull;
+    P.push_relayout = io.push;
     const size_t n = P.launches.size();
-
     const Launch& f = P.launches.front();
-    if (f.kind == StepKind::Elt && f.elt == k::kEltCopy && n >= 2 && plan.steps.at(0).a.buf == in && dense4(f.a) &&
-        f.a.ptr == P.arena + plan.bufs.at(in).offset && same_dims(f.a, f.out) && rows4(f.out)) {
-        P.pull_relayout = true;
-        for (size_t i = 1; i < plan.steps.size(); ++i) {  // nothing else reads the planar input
-            const Step& s = plan.steps[i];
-            for (const VRef* v : {&s.a, &s.b, &s.c, &s.res, &s.cls_in})
-                if (v->buf == in) P.pull_relayout = false;
-        }
-    }
     const Launch& l = P.launches.back();
     const VRef& o = plan.outputs[0];
-    const size_t from = P.pull_relayout ? 1 : 0;
-    P.push_relayout = n > from + 1 && l.kind == StepKind::Elt && l.elt == k::kEltCopy &&
-                      plan.steps.back().out.buf == ob && plan.steps.back().a.buf != ob &&
-                      l.out.ptr == P.arena + plan.bufs.at(ob).offset + o.off && dense4(l.out) &&
-                      same_dims(l.a, l.out) && rows4(l.a) &&
-                      static_cast<int64_t>(P.outputs[0].nbytes) ==
-                          static_cast<int64_t>(sizeof(float)) * l.out.dims[0] * l.out.str[0];
-    if (P.push_relayout)
-        for (size_t i = 0; i + 1 < plan.steps.size(); ++i)
-            for (const VRef* v : {&plan.steps[i].out, &plan.steps[i].a, &plan.steps[i].b, &plan.steps[i].res})
-                if (v->buf == ob) P.push_relayout = false;  // only the copy touches the output
-    const size_t to = P.push_relayout ? n - 1 : n;
+    const size_t from = io.pull ? 1 : 0, to = io.push ? n - 1 : n;
 
     const int64_t N = plan.input_dims.at(0).empty() ? 0 : plan.input_dims[0][0];
     int64_t in_floats = 1;
@@ -1448,26 +1413,10 @@ void Session::plan_io() {
         if (io_slices_ > 0) return std::min<int64_t>(most, io_slices_);
         return pipeline_slices(up_us, down_us, std::min(most, kMaxIoSlices), steps);
     };
-    const bool both = P.pull_relayout && P.push_relayout && l.out.dims[0] == N;
 
     // slices of the batch
-    if (both && N >= 2) {
-        bool ok = true;
-        auto batch_first = [&](const k::View& v) {
-            return v.ptr == nullptr || (v.rank >= 1 && v.dims[0] == N && v.str[0] > 0);
-        };
-        for (size_t i = from; i < to && ok; ++i) {
-            const Launch& b = P.launches[i];
-            if (b.kind == StepKind::ConvMfma)
-                ok = b.group.empty() && b.conv.N == N;
-            else if (b.kind == StepKind::ConvDirect)
-                ok = batch_first(b.direct.x) && batch_first(b.direct.y) && batch_first(b.direct.res);
-            else if (b.kind == StepKind::MaxPoolChain || b.kind == StepKind::MaxPool || b.kind == StepKind::Resize)
-                ok = batch_first(b.out) && batch_first(b.a) && batch_first(b.b) && batch_first(b.c);
-            else
-                ok = false;
-        }
-        const int64_t S = !ok ? 1 : best_slices(N, [&](int64_t n_slices) {
+    if (io.slices == IoSlices::Batch) {
+        const int64_t S = best_slices(N, [&](int64_t n_slices) {
             double us = 0.0;
             for (size_t i = from; i < to; ++i) {
                 const Launch& b = P.launches[i];
@@ -1481,8 +1430,7 @@ void Session::plan_io() {
             }
             return us;
         });
-        ok = ok && S >= 2;
-        for (int64_t i = 0; ok && i < S; ++i) {
+        for (int64_t i = 0; S >= 2 && i < S; ++i) {
             const int64_t n0 = N * i / S, m = N * (i + 1) / S - n0;
             Prepared::IoSlice s;
             s.pull = relayout_of(f.a, f.out, n0, m, 0, f.a.dims[2] * f.a.dims[3], true);
@@ -1506,14 +1454,13 @@ void Session::plan_io() {
             }
             P.io.push_back(std::move(s));
         }
-        if (ok) return;
-        P.io.clear();
+        if (S >= 2) return;
     }
 
     // slices of one image's output rows, each with the input rows it is the
     // first to need (starting at even rows: a Winograd launch's 2x2 tiles
     // stay those of the whole image, and so do the output's bits)
-    if (both && N == 1 && to - from == 1 && P.launches[from].kind == StepKind::ConvMfma) {
+    if (io.slices == IoSlices::Rows) {
         const Launch& b = P.launches[from];
         const k::ConvArgs& c = b.conv;
         const int64_t S = best_slices(static_cast<int64_t>(c.Ho) / 8, [&](int64_t n_slices) {
@@ -1521,7 +1468,7 @@ void Session::plan_io() {
             r.Ho = static_cast<int32_t>((c.Ho + n_slices - 1) / n_slices);
             return launch_us(r, b.tile) * static_cast<double>(n_slices);
         });
-        if (b.group.empty() && c.splits == 1 && !c.up && !c.res && S >= 2) {
+        if (S >= 2) {
             int64_t have = 0;  // input rows of the slices so far
             for (int64_t i = 0; i < S; ++i) {
                 const int64_t r0 = c.Ho * i / S / 2 * 2, r1 = i + 1 < S ? c.Ho * (i + 1) / S / 2 * 2 : c.Ho;
