@@ -321,6 +321,33 @@ void step_views(const Step& s, std::vector<VRef>& rd, std::vector<VRef>& wr) {
     }
 }
 
+// Views that keep the images of a batch of N apart: item n of every view that
+// takes() let pass lies in elements [n * S, (n + 1) * S) of its buffer, with
+// one S per buffer.  An outer dimension of size N alone does not say so: a
+// transposed view's may be channels or rows, and a reshaped and sliced one's
+// parts of images.
+class ImageViews {
+   public:
+    ImageViews(const Plan& p, int64_t N) : N_(N) {
+        for (int32_t b : p.input_bufs) item_[{b, 0}] = p.bufs.at(static_cast<size_t>(b)).elems / N;
+    }
+    bool takes(const VRef& v) {
+        if (v.rank < 1 || v.dims[0] != N_ || v.str[0] <= 0) return false;
+        int64_t lo = v.off, hi = v.off;  // of item 0
+        for (int d = 1; d < v.rank; ++d) {
+            if (v.dims[d] <= 0) return false;
+            const int64_t e = (v.dims[d] - 1) * v.str[d];
+            (e < 0 ? lo : hi) += e;
+        }
+        const int64_t S = item_.emplace(std::make_pair(v.buf, v.aux), v.str[0]).first->second;
+        return S == v.str[0] && lo >= 0 && hi < S;
+    }
+
+   private:
+    int64_t N_;
+    std::map<std::pair<int32_t, int32_t>, int64_t> item_;  // S of a buffer (a weight: buf, aux)
+};
+
 // Whether two views of planned buffers may share an element.  Distinct
 // buffers never do before memory is assigned; two views of one buffer are
 // disjoint when they are slices of one parent along one axis with disjoint
@@ -2008,21 +2035,22 @@ IoShape io_shape(const Plan& p) {
     const size_t to = p.steps.size() - 1;
 
     if (N >= 2) {
-        auto batch_first = [&](const VRef& v) {
-            return v.buf == -1 || (v.rank >= 1 && v.dims[0] == N && v.str[0] > 0);
-        };
-        for (size_t i = from; i < to; ++i) {
+        ImageViews images(p, N);
+        for (size_t i = 0; i < p.steps.size(); ++i) {
             const Step& s = p.steps[i];
-            bool ok = false;
-            if (s.kind == StepKind::ConvMfma)
-                ok = s.group < 0 && s.a.dims[0] == N;
-            else if (s.kind == StepKind::ConvDirect)
-                ok = batch_first(s.a) && batch_first(s.out) && (!s.has_res || batch_first(s.res));
-            else if (s.kind == StepKind::MaxPool || s.kind == StepKind::Resize)
-                ok = batch_first(s.a) && batch_first(s.out);
-            else if (s.kind == StepKind::MaxPoolChain)
-                ok = batch_first(s.a) && batch_first(s.out) && batch_first(s.b) && batch_first(s.c);
-            if (!ok) return io;
+            const bool edge = i < from || i >= to;
+            if (!edge && !(s.kind == StepKind::ConvMfma && s.group < 0) && s.kind != StepKind::ConvDirect &&
+                s.kind != StepKind::MaxPool && s.kind != StepKind::MaxPoolChain && s.kind != StepKind::Resize)
+                return io;
+            if (edge) {
+                rd = {s.a};
+                wr = {s.out};
+            } else {
+                step_views(s, rd, wr);
+            }
+            for (const auto* vs : {&rd, &wr})
+                for (const VRef& v : *vs)
+                    if (!images.takes(v)) return io;
         }
         io.slices = IoSlices::Batch;
     } else if (N == 1 && to - from == 1) {

@@ -50,6 +50,49 @@ def _one_conv(cin, cout, k, s, hw):
     return ys.build_single_conv(cin, cout, k, s, hw, seed=3)[0], (1, cin, hw, hw)
 
 
+def _batch(build, n, c, h, w, out_shape):
+    return _graph(build, (n, c, h, w), out_shape), (n, c, h, w)
+
+
+def _transpose(b, x, perm):
+    return b.node("Transpose", "/t", [x, b.const("/t::perm", np.array(perm, np.float32))])
+
+
+def _pool(b, x):
+    return b.node("MaxPool", "/p", [x], kernel_h=3, kernel_w=3, stride_h=1, stride_w=1, pad_h=1, pad_w=1)
+
+
+def _block(kind, c, h, w, n):
+    def build(b, y):
+        if kind == "c2f":
+            return y.c2f(-1, c, c, 1, True, "block")
+        if kind == "sppf":
+            return y.sppf(-1, c, c, "block")
+        return y.conv(_pool(b, y.conv(-1, c, c, 1, 1, "a")), c, c, 3, 1, "b")
+
+    return _batch(build, n, c, h, w, (n, c, h, w))
+
+
+def _transposed(n, cin, mid, h, w, perm, cout, k, pool=False):
+    """A conv to `mid` channels, a Transpose, optionally a pool, a conv."""
+    dims = [(n, mid, h, w)[i] for i in perm]
+
+    def build(b, y):
+        t = _transpose(b, y.conv(-1, cin, mid, 1, 1, "a"), perm)
+        return y.conv(_pool(b, t) if pool else t, dims[1], cout, k, 1, "b")
+
+    return _batch(build, n, cin, h, w, (dims[0], cout, dims[2], dims[3]))
+
+
+def _half_images(n, c, h, w, first):
+    """N of the 2N half images that a Reshape makes of N images."""
+    def build(b, y):
+        half = b.node("Reshape", "/r", [y.conv(-1, c, c, 1, 1, "a"), b.const("/r::shape", [2 * n, c // 2, h, w])])
+        return y.conv(y.slice(half, first, first + n, 0, "/s"), c // 2, 16, 3, 1, "b")
+
+    return _batch(build, n, c, h, w, (n, 16, h, w))
+
+
 # name: (model and input shape, slices)
 CASES = {
     "conv": (lambda: _one_conv(64, 64, 3, 1, 48), "rows"),
@@ -64,6 +107,19 @@ CASES = {
     "rows 4..48 conv": (lambda: _slice_conv(32, 24, 48, 2, 4, 48), "none"),
     "channels 8..32 conv": (lambda: _slice_conv(32, 24, 48, 1, 8, 32), "none"),
     "two convs rows 0..20": (lambda: _conv_conv(32, 40, 20), "none"),
+    # batches, whose every step keeps the images apart
+    "c2f batch": (lambda: _block("c2f", 64, 20, 24, 4), "batch"),
+    "sppf batch": (lambda: _block("sppf", 64, 12, 20, 3), "batch"),
+    "pool batch": (lambda: _block("pool", 32, 12, 20, 32), "batch"),
+    # an outer dimension of the batch's size that is channels or rows
+    "channels as images": (lambda: _transposed(16, 32, 16, 20, 20, (1, 0, 2, 3), 24, 3), "none"),
+    "channels as images, pool": (lambda: _transposed(16, 32, 16, 20, 20, (1, 0, 2, 3), 24, 3, True), "none"),
+    "channels as images, 1x1": (lambda: _transposed(16, 32, 16, 20, 20, (1, 0, 2, 3), 24, 1), "none"),
+    "rows as images": (lambda: _transposed(20, 32, 48, 20, 16, (2, 1, 0, 3), 24, 3), "none"),
+    "rows and columns swapped": (lambda: _transposed(4, 32, 48, 12, 20, (0, 1, 3, 2), 24, 3), "batch"),
+    # parts of images
+    "first half images": (lambda: _half_images(4, 32, 12, 12, 0), "none"),
+    "last half images": (lambda: _half_images(4, 32, 12, 12, 4), "none"),
 }
 
 
