@@ -446,6 +446,8 @@ PDEFA_EXPORT EngineStatus pdefa_amd_plan_model(const EngineModel* m, const int64
         // as a session plans it: the Detect decode split per anchor range
         const char* so = std::getenv("PDEFA_SPLIT_OUTPUTS");
         opt.split_outputs = !(so && so[0] == '0');
+        // PDEFA_EARLY_HW, where it is set, as a session on a batch takes it
+        if (const char* h = std::getenv("PDEFA_EARLY_HW"); h && shape[0] >= 2) opt.early_hw = std::atoll(h);
         if (const char* g = std::getenv("PDEFA_PLAN_GROUP_ALL"); g && g[0] == '1') {
             // Host-only stand-ins for the device measurements: launch shapes
             // from the cost model, and every group the grouping pass offers

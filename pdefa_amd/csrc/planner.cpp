@@ -1717,33 +1717,29 @@ class Planner {
     }
 
     // Length of the leading run of steps that process each image on its own
-    // (conv and elementwise steps whose every view has the batch N as its
-    // outer dimension, or is broadcast over it) on outputs of at least
-    // early_hw pixels, ending at a grouped launch's end.
+    // (conv and elementwise steps whose views keep the images apart, the
+    // constants aside) on outputs of at least early_hw pixels, ending at a
+    // grouped launch's end.
     int early_prefix() const {
         if (opt_.early_hw <= 0 || plan_.input_dims.empty() || plan_.input_dims[0].empty()) return 0;
         const int64_t N = plan_.input_dims[0][0];
         if (N < 2) return 0;
-        auto batch_view = [&](const VRef& v, bool broadcast_ok) {
-            if (v.buf == -1 || v.buf == kBufWeight) return true;
-            if (v.rank < 1) return false;
-            if (v.dims[0] == N) return v.str[0] > 0 || N == 1;
-            return broadcast_ok && v.dims[0] == 1;
-        };
+        ImageViews images(plan_, N);
+        // a constant is whole from the start, whatever part of it a chunk reads
+        auto operand = [&](const VRef& v) { return v.buf == -1 || v.buf == kBufWeight || images.takes(v); };
         const auto& st = plan_.steps;
         int e = 0;
         for (size_t i = 0; i < st.size(); ++i) {
             const Step& s = st[i];
             bool ok = false;
             if (s.kind == StepKind::ConvMfma || s.kind == StepKind::ConvDirect) {
-                ok = s.out.rank == 4 && s.out.dims[2] * s.out.dims[3] >= opt_.early_hw && batch_view(s.out, false) &&
-                     batch_view(s.a, false) && (!s.has_res || batch_view(s.res, false)) &&
-                     (s.kind != StepKind::ConvMfma || s.up.buf == -1 || batch_view(s.up, false));
+                ok = s.out.rank == 4 && s.out.dims[2] * s.out.dims[3] >= opt_.early_hw && images.takes(s.out) &&
+                     images.takes(s.a) && (!s.has_res || images.takes(s.res)) &&
+                     (s.kind != StepKind::ConvMfma || s.up.buf == -1 || images.takes(s.up));
             } else if (s.kind == StepKind::Elt) {
                 int64_t hw = 1;
                 for (int d = 2; d < s.out.rank; ++d) hw *= s.out.dims[d];
-                ok = s.out.rank >= 3 && hw >= opt_.early_hw && batch_view(s.out, false) && batch_view(s.a, true) &&
-                     batch_view(s.b, true);
+                ok = s.out.rank >= 3 && hw >= opt_.early_hw && images.takes(s.out) && operand(s.a) && operand(s.b);
             }
             if (!ok) break;
             const bool group_continues = s.group >= 0 && i + 1 < st.size() && st[i + 1].group == s.group;

@@ -138,6 +138,20 @@ def test_slices(name, tmp_path):
     assert transfers(native.plan_text(path, list(shape)))[2] == slices
 
 
+# steps that run on chunks of the batch as the input arrives (of CASES' steps:
+# the layout copy, the convs and pools, the layout copy)
+@pytest.mark.parametrize("name,early", [
+    ("c2f batch", 6), ("channels as images", 2), ("channels as images, 1x1", 2), ("rows as images", 2),
+    ("rows and columns swapped", 4), ("first half images", 3), ("last half images", 3),
+])
+def test_early_steps(name, early, tmp_path, monkeypatch):
+    monkeypatch.setenv("PDEFA_EARLY_HW", "1")
+    model, shape = CASES[name][0]()
+    path = os.path.join(tmp_path, "m.engine")
+    ys.save(model, path)
+    assert int(re.search(r"early_steps=(\d+)", native.plan_text(path, list(shape))).group(1)) == early
+
+
 def _run(path, xs, env, monkeypatch):
     for k, v in env.items():
         monkeypatch.setenv(k, v)
@@ -161,8 +175,10 @@ def test_outputs(name, tmp_path, monkeypatch):
     rng = np.random.default_rng(5)
     xs = [rng.standard_normal(shape, dtype=np.float32) for _ in range(2)]
     want = _run(path, xs, {"PDEFA_HIP_GRAPH": "0"}, monkeypatch)
-    for n in (0, 1, 2, 3):
-        print(f"[case] {name} slices {n}", flush=True)
-        got = _run(path, xs + xs[:1], {"PDEFA_IO_SLICES": str(n)} if n else {}, monkeypatch)
-        for g, w in zip(got, want + want[:1]):
+    envs = [{}] + [{"PDEFA_IO_SLICES": str(n)} for n in (1, 2, 3)]
+    if shape[0] % 2 == 0:
+        envs.append({"PDEFA_EARLY_HW": "1"})  # chunks of the batch
+    for env in envs:
+        print(f"[case] {name} {env}", flush=True)
+        for g, w in zip(_run(path, xs + xs[:1], env, monkeypatch), want + want[:1]):
             np.testing.assert_array_equal(g, w)
