@@ -2007,8 +2007,10 @@ IoShape io_shape(const Plan& p) {
     const int64_t N = p.input_dims[0][0];
     const Step& f = p.steps.front();
     const Step& l = p.steps.back();
-    io.pull = f.kind == StepKind::Elt && f.elt == k::kEltCopy && f.a.buf == in && f.a.off == 0 && dense4(f.a) &&
-              dims_of(f.a) == dims_of(f.out) && rows4(f.out);
+    // (the copy reads the input in the input's own shape, not a Slice or a
+    // Reshape of it)
+    io.pull = f.kind == StepKind::Elt && f.elt == k::kEltCopy && f.a.buf == in && f.a.off == 0 &&
+              dims_of(f.a) == p.input_dims[0] && dense4(f.a) && dims_of(f.a) == dims_of(f.out) && rows4(f.out);
     std::vector<VRef> rd, wr;
     for (size_t i = 1; i < p.steps.size(); ++i) {  // nothing else reads the planar input
         step_views(p.steps[i], rd, wr);

@@ -1500,7 +1500,7 @@ void Session::plan_io() {
     Prepared::IoSlice s;
     s.up.width = in_floats;
     s.down.width = out_bytes / static_cast<int64_t>(sizeof(float));
-    if (P.pull_relayout) s.pull = relayout_of(f.a, f.out, 0, N, 0, f.a.dims[2] * f.a.dims[3], true);
+    if (P.pull_relayout) s.pull = relayout_of(f.a, f.out, 0, f.a.dims[0], 0, f.a.dims[2] * f.a.dims[3], true);
     if (P.push_relayout) s.push = relayout_of(l.out, l.a, 0, l.out.dims[0], 0, l.out.dims[2] * l.out.dims[3], false);
     s.body.assign(P.launches.begin() + static_cast<int64_t>(from), P.launches.begin() + static_cast<int64_t>(to));
     P.io.push_back(std::move(s));

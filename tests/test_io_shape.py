@@ -93,6 +93,24 @@ def _half_images(n, c, h, w, first):
     return _batch(build, n, c, h, w, (n, 16, h, w))
 
 
+def _view_concat(n, c, h, w, view):
+    """The input, sliced or reshaped, beside a constant in a concat's
+    channels-last buffer, and a conv of both."""
+    dims = {"image 0": (1, c, h, w), "halves": (2 * n, c // 2, h, w), "whole": (n, c, h, w)}[view]
+
+    def build(b, y):
+        x = -1
+        if view == "image 0":
+            x = y.slice(-1, 0, 1, 0, "/s")
+        elif view == "halves":
+            x = b.node("Reshape", "/r", [-1, b.const("/r::shape", list(dims))])
+        const = np.random.default_rng(4).standard_normal((dims[0], 16, h, w)).astype(np.float32)
+        cat = b.node("Concat", "/c", [x, b.const("/c::const", const)], axis=1)
+        return y.conv(cat, dims[1] + 16, 24, 3, 1, "a")
+
+    return _batch(build, n, c, h, w, (dims[0], 24, h, w))
+
+
 # name: (model and input shape, slices)
 CASES = {
     "conv": (lambda: _one_conv(64, 64, 3, 1, 48), "rows"),
@@ -120,6 +138,12 @@ CASES = {
     # parts of images
     "first half images": (lambda: _half_images(4, 32, 12, 12, 0), "none"),
     "last half images": (lambda: _half_images(4, 32, 12, 12, 4), "none"),
+    # the first copy reads a part of the input, or it in another shape
+    "image 0 of 2": (lambda: _view_concat(2, 16, 20, 20, "image 0"), "none"),
+    "halves of an image": (lambda: _view_concat(1, 32, 20, 20, "halves"), "none"),
+    "halves of images": (lambda: _view_concat(2, 32, 20, 20, "halves"), "none"),
+    "input beside a constant": (lambda: _view_concat(1, 16, 20, 20, "whole"), "none"),
+    "inputs beside a constant": (lambda: _view_concat(2, 16, 20, 20, "whole"), "none"),
 }
 
 
@@ -136,6 +160,19 @@ def test_slices(name, tmp_path):
     path = os.path.join(tmp_path, "m.engine")
     ys.save(model, path)
     assert transfers(native.plan_text(path, list(shape)))[2] == slices
+
+
+@pytest.mark.parametrize("name,pull", [
+    ("conv", 1), ("image 0 of 2", 0), ("halves of an image", 0), ("halves of images", 0), ("input beside a constant", 1),
+    ("inputs beside a constant", 1), ("rows 4..48 conv", 0), ("conv rows 4..48", 1),
+])
+def test_pull(name, pull, tmp_path):
+    """The upload takes the first layout copy's place only where that copy
+    reads the whole input in its own shape."""
+    model, shape = CASES[name][0]()
+    path = os.path.join(tmp_path, "m.engine")
+    ys.save(model, path)
+    assert transfers(native.plan_text(path, list(shape)))[0] == pull
 
 
 # steps that run on chunks of the batch as the input arrives (of CASES' steps:
