@@ -87,7 +87,8 @@ enum ConvTile : int32_t {
     kTile16x32K8W8 = 19,   // 1 wave tile of 16x32, K split in 8
     kTile32x16K8W8 = 20,   // 1 wave tile of 32x16, K split in 8
     // The implicit GEMM on the bf16 matrix cores with each f32 operand split
-    // into three bf16 terms (conv_mfma_tile.hpp); finite weights only
+    // into three bf16 terms (conv_mfma_tile.hpp); for weights that the terms
+    // hold (the planner checks)
     kTileSplit128x128W8 = 21,  // 2x4 waves of 64x32
     kNumConvShapes = 22,   // tile ids (implicit-GEMM, Winograd and split)
 };

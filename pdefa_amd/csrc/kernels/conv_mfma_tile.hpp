@@ -59,6 +59,7 @@ namespace k {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 namespace {
@@ -143,28 +144,23 @@ __device__ __forceinline__ int xcd_tile(int lin, int total) {
 // pass and an upsampled copy (the launchers check).
 constexpr int kEpiPlain = 0, kEpiFix = 1, kEpiUp = 2, kEpiFixOnly = 3;
 
-// x as three bf16 terms whose sum is x: each takes the leading 8 significand
-// bits of what the ones before it leave, by truncation, so every difference
-// is exact and 24 bits are covered; a term is the upper half of its float.
-// A NaN stays one in the terms.  INF: x may be infinite, and goes to the last
-// term alone then, which meets only the leading term of the other operand:
-// the products with it are those of x itself (beside a finite x's other terms
-// an infinite leading one would meet zeros).
-struct SplitTerms {
-    uint32_t t[3];
-};
-template <bool INF>
-__device__ __forceinline__ SplitTerms split_terms(float x) {
-    const bool fin = !INF || __builtin_fabsf(x) < __builtin_inff();
-    const float v = fin ? x : 0.0f;
-    SplitTerms s;
-    s.t[0] = __float_as_uint(v) & 0xffff0000u;
-    const float r = v - __uint_as_float(s.t[0]);
-    s.t[1] = __float_as_uint(r) & 0xffff0000u;
-    const float l = r - __uint_as_float(s.t[1]);
-    s.t[2] = __float_as_uint(fin ? l : x);
-    return s;
+// Two floats as three pairs of bf16 terms (a pair in one word): each term is
+// the leading 8 significand bits of what the ones before it leave, by
+// truncation, so every difference is exact and three terms hold the 24 bits
+// of a normal float.  That is for finite x, and for |x| from 2^-102, below
+// which the last term would be under the smallest normal bf16.
+__device__ __forceinline__ void split_terms(floatx2 x, uint32_t (&t)[3]) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        t[p] = __builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u);
+        x[0] -= __uint_as_float(t[p] << 16);
+        x[1] -= __uint_as_float(t[p] & 0xffff0000u);
+    }
 }
+// The magnitude of x as an unsigned that orders as it does (NaNs highest).
+__device__ __forceinline__ uint32_t magnitude(float x) { return __float_as_uint(x) << 1; }
+constexpr uint32_t kSplitTop = 0x7f800000u << 1;    // infinity
+constexpr uint32_t kSplitSmall = 0x12800000u << 1;  // 2^-90
 
 // One BM x BN output tile (m block bx, n block by) of K split bz of problem a.
 // SPLIT: the products on the bf16 matrix cores (see split_terms).
@@ -351,26 +347,30 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
         for (int i = 0; i < B_ROWS; ++i)
             br[i] = *reinterpret_cast<const floatx4*>(brow[i] + static_cast<int64_t>(kb) * (kConvBN * BK));
     };
-    // the three planes of a float4 chunk of a split row (weights are finite:
-    // the planner checks)
-    auto store_split = [&](auto inf_c, float* row, floatx4 v) {
-        SplitTerms t[4];
+    // the three planes of a float4 chunk of a split row
+    auto store_split = [&](float* row, floatx4 v) {
+        uint32_t lo[3], hi[3];
+        split_terms(floatx2{v[0], v[1]}, lo);
+        split_terms(floatx2{v[2], v[3]}, hi);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = split_terms<decltype(inf_c)::value>(v[e]);
+        for (int p = 0; p < 3; ++p)
+            *reinterpret_cast<uint2*>(row + p * (BK / 2) + cc * 2) = make_uint2(lo[p], hi[p]);
+    };
+    // split tiles: the largest magnitude in this lane's part of its A rows
+    uint32_t a_top[SPLIT ? A_ROWS : 1] = {};
+    auto store_split_a = [&](float* rows, int r, floatx4 v) {
+        store_split(rows + (r0 + ROW_STEP * r) * STRIDE, v);
 #pragma unroll
-        for (int p = 0; p < 3; ++p)  // the upper halves of two words as one
-            *reinterpret_cast<uint2*>(row + p * (BK / 2) + cc * 2) =
-                make_uint2(__builtin_amdgcn_perm(t[1].t[p], t[0].t[p], 0x07060302u),
-                           __builtin_amdgcn_perm(t[3].t[p], t[2].t[p], 0x07060302u));
+        for (int e = 0; e < 4; ++e) a_top[r] = max(a_top[r], magnitude(v[e]));
     };
     auto store_step = [&](int st, const floatx4* ar, const floatx4* br) {
         float* A = As(st, cg);
         float* B = Bs(st, cg);
         if constexpr (SPLIT) {
 #pragma unroll
-            for (int r = 0; r < A_ROWS; ++r) store_split(std::true_type{}, &A[(r0 + ROW_STEP * r) * STRIDE], ar[r]);
+            for (int r = 0; r < A_ROWS; ++r) store_split_a(A, r, ar[r]);
 #pragma unroll
-            for (int i = 0; i < B_ROWS; ++i) store_split(std::false_type{}, &B[(r0 + ROW_STEP * i) * STRIDE], br[i]);
+            for (int i = 0; i < B_ROWS; ++i) store_split(&B[(r0 + ROW_STEP * i) * STRIDE], br[i]);
             return;
         }
 #pragma unroll
@@ -403,64 +403,61 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     // Split step: the products of LDS stage st, and between them the split and
     // the LDS stores of the next step's loads (next: into stage st ^ 1, which
     // no wave reads before the barrier), so that the vector ALU works through
-    // the splits while the matrix core multiplies.  Both 16-wide quarters'
-    // fragments are read ahead of their products.
+    // the splits while the matrix core multiplies.  The fragments of both
+    // 16-wide quarters are read ahead of the products.
     // v_mfma_f32_32x32x16_bf16: lane half h supplies k = 16q + 8h .. +7 of its
     // row.  The six products of terms down to 2^-16 of the leading one; the
-    // dropped ones are below 2^-23 of it.
+    // dropped ones are below 2^-21 of it (each of the two below 2^-22, and
+    // with the product's sign).
     //
     // What bounds it: per 32-wide step of a 128 x 128 tile a SIMD has 1536
-    // cycles of MFMAs, about 1250 of vector ALU (5.5 to 8.5 instructions a
+    // cycles of MFMAs, about 1250 of vector ALU (5.5 to 7 instructions a
     // loaded element) and the CU 1400 of LDS traffic, which overlap only in
     // part (about 3800 measured).  16 x 40x40 images, us against the f32 tile
     // of the launch-shape table: 768 -> 384 1x1 114 / 161 (198 TFLOP/s), 384
     // -> 384 1x1 67 / 88; 16 x 20x20, 1152 -> 576: 62 / 97.  Tried: four
     // waves of 64x64 (140) and 128 x 64 tiles, two workgroups a CU (124);
     // one quarter's fragments at a time (129); the groups of products held in
-    // order by scheduling barriers (122); a wave-uniform branch around the
-    // handling of infinities (219: it spills).
+    // order by scheduling barriers (122); a wave-uniform branch around a
+    // handling of infinities in the terms (219: it spills).
     auto split_step = [&](int st, const floatx4* ar, const floatx4* br, bool next) {
         if constexpr (SPLIT) {
             constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
-            constexpr int CHUNKS = A_ROWS + B_ROWS, KQS = BK / 16, GROUPS = 6 * KQS, FQ = KQS;
+            constexpr int CHUNKS = A_ROWS + B_ROWS, KQS = BK / 16, GROUPS = 6 * KQS;
             const float* Ab = As(st, 0);
             const float* Bb = Bs(st, 0);
             float* An = As(st ^ 1, 0);
             float* Bn = Bs(st ^ 1, 0);
-            bf16x8 av[FQ][TM][3], bv[FQ][TN][3];
-            auto frags = [&](int q) {
+            bf16x8 av[KQS][TM][3], bv[KQS][TN][3];
+#pragma unroll
+            for (int q = 0; q < KQS; ++q)
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
 #pragma unroll
                     for (int tm = 0; tm < TM; ++tm)
-                        av[q % FQ][tm][p] = *reinterpret_cast<const bf16x8*>(
+                        av[q][tm][p] = *reinterpret_cast<const bf16x8*>(
                             &Ab[(wave_m * WM + tm * MB + lcol) * STRIDE + p * (BK / 2) + q * 8 + half * 4]);
 #pragma unroll
                     for (int tn = 0; tn < TN; ++tn)
-                        bv[q % FQ][tn][p] = *reinterpret_cast<const bf16x8*>(
+                        bv[q][tn][p] = *reinterpret_cast<const bf16x8*>(
                             &Bb[(wave_n * WN + tn * MB + lcol) * STRIDE + p * (BK / 2) + q * 8 + half * 4]);
                 }
-            };
-#pragma unroll
-            for (int q = 0; q + 1 < FQ; ++q) frags(q);
             static_for<GROUPS>([&](auto gc) {
                 constexpr int G = decltype(gc)::value, q = G / 6, P = G % 6;
-                if (P == 0 && q + FQ - 1 < KQS) frags(q + FQ - 1);
 #pragma unroll
                 for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
                     for (int tn = 0; tn < TN; ++tn) {
                         AccT& c = P == 5 ? acc[tm][tn] : low[tm][tn];
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[q % FQ][tm][PA[P]], bv[q % FQ][tn][PB[P]], c, 0, 0,
-                                                                    0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[q][tm][PA[P]], bv[q][tn][PB[P]], c, 0, 0, 0);
                     }
                 if (next)
 #pragma unroll
                     for (int i = CHUNKS * G / GROUPS; i < CHUNKS * (G + 1) / GROUPS; ++i) {
                         if (i < A_ROWS)
-                            store_split(std::true_type{}, &An[(r0 + ROW_STEP * i) * STRIDE], ar[i]);
+                            store_split_a(An, i, ar[i]);
                         else
-                            store_split(std::false_type{}, &Bn[(r0 + ROW_STEP * (i - A_ROWS)) * STRIDE], br[i - A_ROWS]);
+                            store_split(&Bn[(r0 + ROW_STEP * (i - A_ROWS)) * STRIDE], br[i - A_ROWS]);
                     }
             });
         }
@@ -580,6 +577,31 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     });
 
     if constexpr (SPLIT) {
+        // A tile with an A row that the terms do not hold goes to the f32
+        // kernel as a whole: one with infinities or NaNs, or a row of nothing
+        // but tiny values (beside one of 2^-90 the terms that a smaller value
+        // may lose are below 2^-36 of it).  The stages are free after the
+        // loop's last barrier.
+        static_assert(CH == 8, "a row's chunks lie in neighbouring lanes");
+        bool out = false;
+#pragma unroll
+        for (int r = 0; r < A_ROWS; ++r) {
+            uint32_t t = a_top[r];
+#pragma unroll
+            for (int d = 1; d < CH; d *= 2) t = max(t, static_cast<uint32_t>(__shfl_xor(static_cast<int>(t), d)));
+            out |= t >= kSplitTop || (t != 0 && t < kSplitSmall);
+        }
+        int* s_out = reinterpret_cast<int*>(smem);  // one flag a wave
+        const uint64_t any = __ballot(out);
+        if (lane == 0) s_out[wave] = any != 0;
+        __syncthreads();
+        int wg_out = 0;
+        for (int w = 0; w < static_cast<int>(blockDim.x) / 64; ++w) wg_out |= s_out[w];
+        if (wg_out) {
+            __syncthreads();  // the flags are read before the stages are filled again
+            conv_tile<BM, BN, WM, WN, KG, PF, VEC, EPI, false>(a, bx, by, bz, grp);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll

@@ -1103,7 +1103,7 @@ class Planner {
             }
             if (k::is_wino_tile(opt_.force_tile)) {
                 if (wino) ls = {opt_.force_tile, 1, static_cast<int>((K + k::kConvBK - 1) / k::kConvBK)};
-            } else if (k::is_gemm_tile(opt_.force_tile) || (k::is_split_tile(opt_.force_tile) && s.vec && G == 1 && finite_weight(n.inputs[1]))) {
+            } else if (k::is_gemm_tile(opt_.force_tile) || (k::is_split_tile(opt_.force_tile) && s.vec && G == 1 && splittable_weight(n.inputs[1]))) {
                 const int kg = k::conv_tile_shape(opt_.force_tile).kg;
                 const int steps_total = static_cast<int>((K + k::kConvBK - 1) / k::kConvBK + kg - 1) / kg;
                 const int want = std::max(1, std::min(opt_.force_splits, steps_total));
@@ -1675,16 +1675,20 @@ class Planner {
         for (const VRef& v : plan_.outputs) check(v, -1, "graph output");
     }
 
-    // Every value of constant r (a conv's weight) is finite: the split tile
-    // handles infinite inputs only.
-    bool finite_weight(int32_t r) const {
+    // The split tile's terms hold constant r (a conv's weight): every output
+    // channel is zero or has a weight of at least 2^-90 (as the tile asks of
+    // its input's rows), and none of 2^127 or more, infinite or NaN.
+    bool splittable_weight(int32_t r) const {
         const HostTensor& w = m_.weights.at(static_cast<size_t>(-1000 - r));
-        if (w.dtype != kF32) return false;
+        if (w.dtype != kF32 || w.rank < 1 || w.dims[0] < 1) return false;
         const uint32_t* v = static_cast<const uint32_t*>(w.data);
-        const int64_t n = w.numel();
-        uint32_t bad = 0;
-        for (int64_t i = 0; i < n; ++i) bad |= (v[i] & 0x7f800000u) == 0x7f800000u;
-        return bad == 0;
+        const int64_t per = w.numel() / w.dims[0];
+        for (int64_t co = 0; co < w.dims[0]; ++co) {
+            uint32_t top = 0;
+            for (int64_t i = 0; i < per; ++i) top = std::max(top, v[co * per + i] & 0x7fffffffu);
+            if (top >= 0x7f000000u || (top != 0 && top < 0x12800000u)) return false;
+        }
+        return true;
     }
 
     // Long implicit GEMMs to the split tile (PlanOptions::split_terms): those
@@ -1708,7 +1712,7 @@ class Planner {
             const int64_t K = s.a.dims[1] * s.KH * s.KW;
             const int64_t cols = (cout + 127) / 128;
             if (K < 768 || (M + 127) / 128 * cols < 128 || 10 * cout < 9 * 128 * cols) continue;
-            if (!finite_weight(m_.nodes[s.node].inputs[1])) continue;
+            if (!splittable_weight(m_.nodes[s.node].inputs[1])) continue;
             s.tile = k::kTileSplit128x128W8;
             s.splits = 1;
             s.kt_per_split = static_cast<int32_t>((K + k::kConvBK - 1) / k::kConvBK);

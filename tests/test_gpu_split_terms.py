@@ -96,3 +96,91 @@ def test_split_rule(tmp_path, monkeypatch):
     w = next(v for v in model.weights if v.size == 768 * 256)
     w.reshape(-1)[77] = np.inf
     assert "split128x128w8" not in plan()
+
+
+def _engine(model, path):
+    ys.save(model, path)
+    return path
+
+
+@pytest.mark.parametrize("bits", [0x7F800001, 0x7F80FFFF, 0xFF800001, 0xFF80FFFF, 0x7FC00000, 0xFFFFFFFF, 0x7F800000,
+                                  0xFF800000])
+def test_split_tile_special_values(bits, tmp_path, monkeypatch):
+    """NaNs of every payload and infinities give the f32 tile's bits in the
+    tile that they reach (here all of it)."""
+    print(f"[case] split {bits:#x}", flush=True)
+    path = _engine(ys.build_single_conv(64, 128, 1, 1, 8, seed=3, silu=False)[0], os.path.join(tmp_path, "c.engine"))
+    x = np.random.default_rng(2).standard_normal((1, 64, 8, 8)).astype(np.float32)
+    x.view(np.uint32)[0, 5, 3, 3] = bits
+    got, f32 = (_run(path, x, t, monkeypatch) for t in ("split128x128w8", "128x128w8"))
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(f32))
+    np.testing.assert_array_equal(got[~np.isnan(got)], f32[~np.isnan(f32)])
+    if bits & 0x7FFFFFFF > 0x7F800000:
+        assert np.isnan(got[0, :, 3, 3]).all()
+
+
+@pytest.mark.parametrize("scale", [1e-27, 1e-30, 1e-33, 1e-36, 1e-39])
+@pytest.mark.parametrize("rows", ["all", "one"])
+def test_split_tile_tiny_rows(scale, rows, tmp_path, monkeypatch):
+    """An input whose values are all tiny (or those of one pixel), where the
+    terms run out of exponents, is no further off than with the f32 tile."""
+    print(f"[case] split tiny {scale} {rows}", flush=True)
+    model = ys.build_single_conv(256, 128, 1, 1, 16, seed=3, silu=False)[0]
+    model.weights[1][:] = 0  # no bias: the products alone
+    path = _engine(model, os.path.join(tmp_path, "c.engine"))
+    x = np.random.default_rng(1).standard_normal((1, 256, 16, 16)).astype(np.float32)
+    part = (0, slice(None), 9, 3) if rows == "one" else (0,)
+    x[part] *= np.float32(scale)
+    want = np.einsum("oi,ihw->ohw", model.weights[0][:, :, 0, 0].astype(np.float64), x[0].astype(np.float64))
+    got, f32 = (_run(path, x, t, monkeypatch)[0].astype(np.float64) for t in ("split128x128w8", "128x128w8"))
+
+    def err(y):
+        d, r = (y - want)[part[1:]], want[part[1:]]
+        return np.linalg.norm(d / scale) / np.linalg.norm(r / scale)
+
+    assert err(got) <= err(f32)
+
+
+@pytest.mark.parametrize("splits", [2, 3])
+def test_split_tile_in_k_parts(splits, tmp_path, monkeypatch):
+    """PDEFA_CONV_SPLITS with the split tile: the K parts' sums."""
+    print(f"[case] split {splits} parts", flush=True)
+    path = _engine(ys.build_single_conv(200, 140, 3, 2, 33, seed=3)[0], os.path.join(tmp_path, "c.engine"))
+    x = np.random.default_rng(2).standard_normal((2, 200, 33, 33)).astype(np.float32)
+    whole = _run(path, x, "split128x128w8", monkeypatch)
+    x[1, 3, 4, 4] = np.nan  # one part of one tile goes to the f32 kernel
+    monkeypatch.setenv("PDEFA_CONV_SPLITS", str(splits))
+    got = _run(path, x, "split128x128w8", monkeypatch)
+    # K = 1800 products of magnitude about 0.1, rounded to 2^-24 of the sum
+    # some K / 16 times in either order
+    np.testing.assert_allclose(got[0], whole[0], rtol=2e-5, atol=2e-5)
+    assert np.isnan(got[1]).any() and np.isfinite(got[1]).any()
+
+
+def test_split_rule_weights(tmp_path, monkeypatch):
+    """An output channel of tiny weights, or a huge one, keeps the layer on
+    the f32 tiles; channels of zeros and a tiny weight beside others do not."""
+    print("[case] split rule weights", flush=True)
+    x = np.random.default_rng(4).standard_normal((1, 768, 96, 96)).astype(np.float32)
+    path = os.path.join(tmp_path, "c.engine")
+
+    def split(change):
+        model = ys.build_single_conv(768, 256, 1, 1, 96, seed=3)[0]
+        change(model.weights[0])
+        eng = native.Engine(_engine(model, path))
+        try:
+            eng.run(x)
+            return "tile=split128x128w8" in eng.plan()
+        finally:
+            eng.close()
+
+    def set_to(at, value):
+        def change(w):
+            w[at] = value
+        return change
+
+    assert split(set_to(7, 0.0))
+    assert split(set_to((7, 5), 1e-40))
+    assert not split(set_to(7, 1e-30))
+    assert not split(set_to((7, 5), 3e38))
+    assert not split(set_to((7, 5), np.nan))
