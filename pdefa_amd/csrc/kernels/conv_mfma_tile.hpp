@@ -60,6 +60,7 @@ namespace k {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 namespace {
@@ -145,21 +146,21 @@ __device__ __forceinline__ int xcd_tile(int lin, int total) {
 constexpr int kEpiPlain = 0, kEpiFix = 1, kEpiUp = 2, kEpiFixOnly = 3;
 
 // Two floats as three pairs of bf16 terms (a pair in one word): each term is
-// the leading 8 significand bits of what the ones before it leave, by
-// truncation, so every difference is exact and three terms hold the 24 bits
-// of a normal float.  That is for finite x, and for |x| from 2^-102, below
-// which the last term would be under the smallest normal bf16.
+// what the ones before it leave, rounded to the nearest, so every difference
+// is exact and three terms of 8 bits hold the 24 of a normal float.  That is
+// for |x| from 2^-102, below which the last term would be under the smallest
+// normal bf16, to 2^128 - 2^119, from which the first one rounds to infinity.
 __device__ __forceinline__ void split_terms(floatx2 x, uint32_t (&t)[3]) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-        t[p] = __builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u);
+        t[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
         x[0] -= __uint_as_float(t[p] << 16);
         x[1] -= __uint_as_float(t[p] & 0xffff0000u);
     }
 }
 // The magnitude of x as an unsigned that orders as it does (NaNs highest).
 __device__ __forceinline__ uint32_t magnitude(float x) { return __float_as_uint(x) << 1; }
-constexpr uint32_t kSplitTop = 0x7f800000u << 1;    // infinity
+constexpr uint32_t kSplitTop = 0x7f7f8000u << 1;     // 2^128 - 2^119
 constexpr uint32_t kSplitSmall = 0x12800000u << 1;  // 2^-90
 
 // One BM x BN output tile (m block bx, n block by) of K split bz of problem a.
@@ -406,20 +407,25 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     // the splits while the matrix core multiplies.  The fragments of both
     // 16-wide quarters are read ahead of the products.
     // v_mfma_f32_32x32x16_bf16: lane half h supplies k = 16q + 8h .. +7 of its
-    // row.  The six products of terms down to 2^-16 of the leading one; the
-    // dropped ones are below 2^-21 of it (each of the two below 2^-22, and
-    // with the product's sign).
+    // row.  The six products of terms down to 2^-16 of the leading one.  Each
+    // of the two dropped next ones is at most 2^-25 of a product of two values
+    // just above powers of two, of either sign: together as much as one f32
+    // rounding at the very most.  Error (2-norm against 64 bits, split / f32
+    // tile): 768 -> 384 1x1 on dense inputs 1.5e-7 / 5.0e-7; on pixels of one
+    // channel, where f32 rounds once, 2.60e-8 / 2.53e-8.  With all eight
+    // products that is 2.53e-8 too, at 125 us for the 108 below.
     //
     // What bounds it: per 32-wide step of a 128 x 128 tile a SIMD has 1536
-    // cycles of MFMAs, about 1250 of vector ALU (5.5 to 7 instructions a
-    // loaded element) and the CU 1400 of LDS traffic, which overlap only in
-    // part (about 3800 measured).  16 x 40x40 images, us against the f32 tile
-    // of the launch-shape table: 768 -> 384 1x1 114 / 161 (198 TFLOP/s), 384
-    // -> 384 1x1 67 / 88; 16 x 20x20, 1152 -> 576: 62 / 97.  Tried: four
-    // waves of 64x64 (140) and 128 x 64 tiles, two workgroups a CU (124);
-    // one quarter's fragments at a time (129); the groups of products held in
-    // order by scheduling barriers (122); a wave-uniform branch around a
-    // handling of infinities in the terms (219: it spills).
+    // cycles of MFMAs, about 1000 of vector ALU (5.5 instructions a loaded
+    // element, 7 for A's with the row magnitudes) and the CU 1400 of LDS
+    // traffic, which overlap only in part (about 3800 measured).  16 x 40x40
+    // images, us against the f32 tile of the launch-shape table: 768 -> 384
+    // 1x1 108 / 140 (210 TFLOP/s), 384 -> 384 1x1 66 / 79; 16 x 20x20, 1152
+    // -> 576: 63 / 85.  Tried, against 114 for the first of these with the
+    // infinities handled in truncated terms: four waves of 64x64 (140) and
+    // 128 x 64 tiles, two workgroups a CU (124); one quarter's fragments at a
+    // time (129); the groups of products held in order by scheduling barriers
+    // (122); a wave-uniform branch around that handling (219: it spills).
     auto split_step = [&](int st, const floatx4* ar, const floatx4* br, bool next) {
         if constexpr (SPLIT) {
             constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
@@ -578,10 +584,10 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
 
     if constexpr (SPLIT) {
         // A tile with an A row that the terms do not hold goes to the f32
-        // kernel as a whole: one with infinities or NaNs, or a row of nothing
-        // but tiny values (beside one of 2^-90 the terms that a smaller value
-        // may lose are below 2^-36 of it).  The stages are free after the
-        // loop's last barrier.
+        // kernel as a whole: one with infinities, NaNs or values that round
+        // to an infinity, or a row of nothing but tiny values (beside one of
+        // 2^-90 the terms that a smaller value may lose are below 2^-36 of
+        // it).  The stages are free after the loop's last barrier.
         static_assert(CH == 8, "a row's chunks lie in neighbouring lanes");
         bool out = false;
 #pragma unroll

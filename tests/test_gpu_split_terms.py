@@ -45,7 +45,7 @@ def test_split_tile(cin, cout, k, s, hw, scale, tmp_path, monkeypatch):
     def err(y):
         return np.linalg.norm(y - want) / np.linalg.norm(want)
 
-    # terms: the dropped products are below 2^-23 of each product, and the
+    # terms: the dropped products are at most 2^-24 of each product, and the
     # K / 16 additions of the leading ones round by 2^-24 of the running sum
     K = cin * k * k
     assert err(got) <= 2.0**-23 + np.sqrt(K / 16 + 1) * 2.0**-24 * 2
@@ -104,10 +104,10 @@ def _engine(model, path):
 
 
 @pytest.mark.parametrize("bits", [0x7F800001, 0x7F80FFFF, 0xFF800001, 0xFF80FFFF, 0x7FC00000, 0xFFFFFFFF, 0x7F800000,
-                                  0xFF800000])
+                                  0xFF800000, 0x7F7FFFFF, 0xFF7F8000])
 def test_split_tile_special_values(bits, tmp_path, monkeypatch):
-    """NaNs of every payload and infinities give the f32 tile's bits in the
-    tile that they reach (here all of it)."""
+    """NaNs of every payload, infinities and the largest finite values give
+    the f32 tile's bits in the tile that they reach (here all of it)."""
     print(f"[case] split {bits:#x}", flush=True)
     path = _engine(ys.build_single_conv(64, 128, 1, 1, 8, seed=3, silu=False)[0], os.path.join(tmp_path, "c.engine"))
     x = np.random.default_rng(2).standard_normal((1, 64, 8, 8)).astype(np.float32)
@@ -184,3 +184,33 @@ def test_split_rule_weights(tmp_path, monkeypatch):
     assert not split(set_to(7, 1e-30))
     assert not split(set_to((7, 5), 3e38))
     assert not split(set_to((7, 5), np.nan))
+
+
+@pytest.mark.parametrize("x_bits", [0x3F80FFFF, 0x3F80FF7F, 0x3F808080, 0x3F80807F, 0x3FFFFFFF, None])
+def test_split_tile_single_products(x_bits, tmp_path, monkeypatch):
+    """Pixels of one channel, so that every output is one product, with the
+    significands whose terms leave the most out (truncated terms: 2^-21 of the
+    product, always towards zero)."""
+    print(f"[case] split single {x_bits}", flush=True)
+    model = ys.build_single_conv(256, 256, 1, 1, 16, seed=3, silu=False)[0]
+    w = model.weights[0]
+    model.weights[1][:] = 0
+    rng = np.random.default_rng(1)
+    x = np.zeros((1, 256, 16, 16), np.float32)
+    if x_bits is None:
+        x[0, np.arange(256), np.arange(256) // 16, np.arange(256) % 16] = rng.standard_normal(256)
+    else:
+        v = np.uint32(x_bits).view(np.float32)
+        x[0, np.arange(256), np.arange(256) // 16, np.arange(256) % 16] = v
+        w[:] = np.where(rng.random(w.shape) < 0.5, v, -v)
+        w[::2] *= (rng.integers(1 << 23, 1 << 24, w[::2].shape) / (1 << 23)).astype(np.float32)
+    path = _engine(model, os.path.join(tmp_path, "c.engine"))
+    want = np.einsum("oi,ihw->ohw", w[:, :, 0, 0].astype(np.float64), x[0].astype(np.float64))
+    got = _run(path, x, "split128x128w8", monkeypatch)[0].astype(np.float64)
+    rel = (got - want) / np.abs(want)
+    # two dropped products of 2^-25 each, the sum's last rounding, and the
+    # low sum's (six of 2^-24 of 2^-7)
+    assert np.abs(rel).max() <= 2.0**-24 * (1 + 1 + 6 / 128)
+    # centred: over random significands the mean error is far below the largest
+    if x_bits is None:
+        assert abs((rel * np.sign(want)).mean()) <= 2.0**-29
