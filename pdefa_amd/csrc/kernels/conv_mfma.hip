@@ -200,7 +200,8 @@ void check_conv(const ConvArgs& a, const ConvTileShape& sh, bool vec) {
     if (a.ktiles != (a.K + BK - 1) / BK) fail("ktiles mismatch");
     const int64_t M = static_cast<int64_t>(a.N) * a.Ho * a.Wo;
     if (a.groups < 1) fail("groups < 1");
-    if (a.row0 < 0 || a.row0 + static_cast<int64_t>(a.Ho) >= (int64_t{1} << 24)) fail("output rows");
+    // (the padding seen from row0 is an int32)
+    if (a.row0 < 0 || a.row0 * static_cast<int64_t>(a.sh) >= (int64_t{1} << 30)) fail("output rows");
     if (a.row0 > 0 && a.splits != 1) fail("split-K takes whole images");
     if (M * std::max(a.Cout, 1) * a.groups >= (int64_t{1} << 31)) fail("M * Cout too large");
     if (a.groups > 1 && a.w_group < packed_weight_elems(a.Cout, a.K)) fail("packed weights per group too small");

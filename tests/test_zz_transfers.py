@@ -90,6 +90,18 @@ def test_matmul_transfers(m, k, n):
         np.testing.assert_allclose(out.numpy(), want, rtol=0, atol=k * 2.0**-24 * 4 + 1e-6)
 
 
+def test_matmul_of_many_rows():
+    """2^24 rows and more in one piece (B is too small to be page-locked, so
+    the product is never sliced)."""
+    m, k, n = (1 << 24) + 5, 4, 4
+    print(f"[case] matmul {m}x{k}x{n}", flush=True)
+    rng = np.random.default_rng(9)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    got = native.matmul(a, b)
+    for rows in (slice(0, 1000), slice(m - 1000, m)):
+        np.testing.assert_allclose(got[rows], a[rows].astype(np.float64) @ b.astype(np.float64), rtol=0, atol=k * 2.0**-24 * 16)
+
+
 def test_matmul_into_its_own_operand():
     from pdefa_amd import pdefa as api
 
