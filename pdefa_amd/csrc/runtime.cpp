@@ -1654,6 +1654,7 @@ void Session::run() {
         return a < h + prep_->outputs[0].nbytes && h < a + inputs_[0]->nbytes;
     };
     const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged() && !in_output();
+    last_io_ = io ? static_cast<int32_t>(prep_->io.size()) : 0;
     if (!segmented && !io) upload_inputs();  // run_segments uploads (by slices) itself
     if (per_step) {
         std::vector<double> ms;
@@ -1805,7 +1806,13 @@ void Session::step_stats(int32_t iters, std::vector<double>& ms, std::vector<int
     }
 }
 
-std::string Session::plan_text() const { return prep_ ? describe_plan(*model_, prep_->plan) : std::string(); }
+std::string Session::plan_text() const {
+    if (!prep_) return std::string();
+    std::ostringstream os;
+    os << describe_plan(*model_, prep_->plan) << "io slices=" << prep_->io.size() << " pull_direct=" << prep_->pull_direct
+       << " push_direct=" << prep_->push_direct << " last_run=" << last_io_ << "\n";
+    return os.str();
+}
 
 void Session::read_conv_input(const std::string& node, std::vector<float>& dst, int64_t dims[4]) {
     if (!keep_tensors_) throw std::runtime_error("tensors are not kept: create the session with PDEFA_KEEP_TENSORS=1");
@@ -2003,6 +2010,24 @@ void matmul_sliced(const MatmulLayout& L, MatmulScratch& sc, const MatmulHost& h
 
 }  // namespace
 
+static int64_t matmul_slices(const MatmulLayout& L, int64_t M, int64_t K, int64_t N) {
+    return pipeline_slices(static_cast<double>(M * K) / kLinkFloatsPerUs, static_cast<double>(M * N) / kLinkFloatsPerUs,
+                           std::min<int64_t>(kMatmulSlices, M / 256), [&](int64_t n) {
+                               k::ConvArgs c;
+                               c.N = c.Wo = c.groups = 1;
+                               c.Ho = static_cast<int32_t>((M + n - 1) / n);
+                               c.Cout = static_cast<int32_t>(N);
+                               c.K = static_cast<int32_t>(K);
+                               c.splits = L.ls.splits;
+                               return launch_us(c, L.ls.tile) * static_cast<double>(n);
+                           });
+}
+
+int64_t matmul_slices(int64_t M, int64_t K, int64_t N) {
+    if (M <= 0 || K <= 0 || N <= 0) return 1;
+    return matmul_slices(matmul_layout(M, K, N), M, K, N);
+}
+
 void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {
     if (!device_available()) throw std::runtime_error("no HIP device available for ops_matmul");
     if (M <= 0 || K <= 0 || N <= 0) return;
@@ -2019,20 +2044,8 @@ void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {
     }
     // slices need page-locked operands, and a C apart from A (a slice of C
     // goes down while later slices of A go up)
-    int64_t slices = 1;
     const bool apart = h.C + M * N <= h.A || h.A + M * K <= h.C;
-    if (h.a_pinned && h.b_pinned && h.c_pinned && apart)
-        slices = pipeline_slices(static_cast<double>(M * K) / kLinkFloatsPerUs,
-                                 static_cast<double>(M * N) / kLinkFloatsPerUs,
-                                 std::min<int64_t>(kMatmulSlices, M / 256), [&](int64_t n) {
-                                     k::ConvArgs c;
-                                     c.N = c.Wo = c.groups = 1;
-                                     c.Ho = static_cast<int32_t>((M + n - 1) / n);
-                                     c.Cout = static_cast<int32_t>(N);
-                                     c.K = static_cast<int32_t>(K);
-                                     c.splits = L.ls.splits;
-                                     return launch_us(c, L.ls.tile) * static_cast<double>(n);
-                                 });
+    const int64_t slices = h.a_pinned && h.b_pinned && h.c_pinned && apart ? matmul_slices(L, M, K, N) : 1;
     if (slices > 1)
         matmul_sliced(L, sc, h, M, K, N, slices);
     else

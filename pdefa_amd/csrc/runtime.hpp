@@ -260,6 +260,7 @@ class Session {
     hipStream_t copy_in_ = nullptr;          // input slices uploaded while earlier chunks compute
     int input_chunks_ = 2;                   // PDEFA_INPUT_CHUNKS (<= 1: the input goes up whole)
     int io_slices_ = 0;                      // PDEFA_IO_SLICES: at most this many slices (0: by size)
+    int32_t last_io_ = 0;                    // slices of the last run (run_io; 0: another path)
     int64_t early_hw_ = 80 * 80;             // PDEFA_EARLY_HW: smallest map the early steps produce
     bool concurrent_ = true;
     std::vector<const HostTensor*> inputs_;
@@ -285,6 +286,9 @@ struct MatmulHost {
 
 // C = A @ B on the device (the ops_matmul path).
 void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N);
+
+// Row slices that device_matmul cuts a product of page-locked operands into.
+int64_t matmul_slices(int64_t M, int64_t K, int64_t N);
 
 // The same product with its device buffers (A, B, packed B, bias, C, split-K
 // partials) in the static scratch array instead of allocated memory; throws

@@ -3,7 +3,9 @@ sliced runs (PDEFA_IO_SLICES) give the bits of the same program run without
 either (PDEFA_HIP_GRAPH=0: upload, every step, download).  The products here
 grow ops_matmul's scratch, so this file runs after test_zz_no_alloc, which
 watches it grow."""
+import ctypes as C
 import os
+import re
 
 import numpy as np
 import pytest
@@ -28,7 +30,7 @@ def _run(path, xs, env, monkeypatch):
     try:
         eng = native.Engine(path)
         try:
-            return [eng.run(x)[0].copy() for x in xs]
+            return [eng.run(x)[0].copy() for x in xs], eng.plan()
         finally:
             eng.close()
     finally:
@@ -36,16 +38,28 @@ def _run(path, xs, env, monkeypatch):
             monkeypatch.delenv(k)
 
 
-def _check(model, shape, tmp_path, monkeypatch, slices):
+def _check(model, shape, tmp_path, monkeypatch, slices, kind, most, direct):
+    """kind: the slices of the plan, `most` of them at the most; direct: whether
+    kernels move the unsliced program's input and output on host memory."""
     path = os.path.join(tmp_path, "m.engine")
     ys.save(model, path)
     rng = np.random.default_rng(5)
     xs = [rng.standard_normal(shape, dtype=np.float32) for _ in range(2)]
-    want = _run(path, xs, {"PDEFA_HIP_GRAPH": "0"}, monkeypatch)
+    want, plan = _run(path, xs, {"PDEFA_HIP_GRAPH": "0"}, monkeypatch)
     assert not np.array_equal(want[0], want[1])
+    assert " last_run=0" in plan
     for s in slices:
         print(f"[case] {shape} slices {s}", flush=True)
-        got = _run(path, xs + xs[:1], {"PDEFA_IO_SLICES": str(s)} if s else {}, monkeypatch)
+        got, plan = _run(path, xs + xs[:1], {"PDEFA_IO_SLICES": str(s)} if s else {}, monkeypatch)
+        if kind == "rows" and not re.search(r"conv_mfma\(\S*,splits=1,", plan):
+            kind = "none"  # the launch shape timed for it splits K
+        assert f"transfers pull=1 push=1 slices={kind}\n" in plan
+        ran, pull, push, last = map(int, re.search(
+            r"io slices=(\d+) pull_direct=(\d) push_direct=(\d) last_run=(\d+)", plan).groups())
+        assert last == ran
+        if s:
+            assert ran == (1 if kind == "none" else max(1, min(s, most)))
+        assert (pull, push) == (int(direct and ran == 1),) * 2
         for g, w in zip(got, want + want[:1]):
             np.testing.assert_array_equal(g, w)
 
@@ -60,24 +74,32 @@ def _check(model, shape, tmp_path, monkeypatch, slices):
 ])
 def test_single_conv_transfers(cin, cout, k, s, hw, tmp_path, monkeypatch):
     model = ys.build_single_conv(cin, cout, k, s, hw, seed=3)[0]
-    _check(model, (1, cin, hw, hw), tmp_path, monkeypatch, [0, 1, 2, 3, 8])
+    _check(model, (1, cin, hw, hw), tmp_path, monkeypatch, [0, 1, 2, 3, 8], "rows", ((hw - 1) // s + 1) // 8, True)
 
 
 @pytest.mark.parametrize("kind,c,h,w,batch", [
     ("c2f", 64, 20, 24, 5), ("c2f", 96, 13, 11, 2), ("sppf", 64, 21, 20, 3), ("scdown", 64, 22, 22, 4),
 ])
 def test_block_transfers(kind, c, h, w, batch, tmp_path, monkeypatch):
-    _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8])
+    _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8], "batch", batch, True)
+
+
+def _matmul_slices(m, k, n):
+    out = C.c_int64()
+    native.check(native.lib().pdefa_amd_matmul_slices(m, k, n, C.byref(out)), "pdefa_amd_matmul_slices")
+    return out.value
 
 
 # Row counts around the slice rule's smallest slice, a remainder row per slice,
 # K % 4 != 0 (4-byte operand loads), products below and above the sizes from
 # which operands are page-locked and sliced, and C in A's memory (never sliced).
-@pytest.mark.parametrize("m,k,n", [(1, 5, 7), (300, 260, 300), (512, 512, 512), (2049, 1023, 1030), (3001, 2047, 601)])
-def test_matmul_transfers(m, k, n):
+@pytest.mark.parametrize("m,k,n,slices", [(1, 5, 7, 1), (300, 260, 300, 1), (512, 512, 512, 1), (2049, 1023, 1030, 3),
+                                          (3001, 2047, 601, 2), (3001, 2047, 1733, 4)])
+def test_matmul_transfers(m, k, n, slices):
     from pdefa_amd import pdefa as api
 
     print(f"[case] matmul {m}x{k}x{n}", flush=True)
+    assert _matmul_slices(m, k, n) == slices
     rng = np.random.default_rng(7)
     for _ in range(2):
         a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
