@@ -141,10 +141,6 @@ PDEFA_EXPORT EngineStatus pdefa_amd_ops_matmul_noalloc(const EngineTensor* a, co
  * process. */
 PDEFA_EXPORT EngineStatus pdefa_amd_tune_stats(int64_t* measured, int64_t* from_table);
 
-/* *slices = the row slices that engine_ops_matmul cuts an [m, k] x [k, n]
- * product of page-locked operands into, whose copies overlap (1: none). */
-PDEFA_EXPORT EngineStatus pdefa_amd_matmul_slices(int64_t m, int64_t k, int64_t n, int64_t* slices);
-
 /* Pre-pack cache files read (*read) and written (*written) by this process.
  * With PDEFA_PACK_CACHE=1 in the environment, a model loaded from an .engine
  * file keeps its packed conv weight layouts (implicit GEMM, direct and

@@ -513,15 +513,6 @@ PDEFA_EXPORT EngineStatus pdefa_amd_tune_stats(int64_t* measured, int64_t* from_
     return ENGINE_OK;
 }
 
-PDEFA_EXPORT EngineStatus pdefa_amd_matmul_slices(int64_t m, int64_t k, int64_t n, int64_t* slices) {
-    if (!slices) return ENGINE_ERR_NULL_PTR;
-    return guarded([&] {
-        clear_error();
-        *slices = pdefa::matmul_slices(m, k, n);
-        return ENGINE_OK;
-    });
-}
-
 PDEFA_EXPORT EngineStatus pdefa_amd_pack_cache_stats(int64_t* read, int64_t* written) {
     if (!read || !written) return ENGINE_ERR_NULL_PTR;
     pdefa::pack_cache_stats(*read, *written);

@@ -2010,7 +2010,11 @@ void matmul_sliced(const MatmulLayout& L, MatmulScratch& sc, const MatmulHost& h
 
 }  // namespace
 
+// Row slices of a product of page-locked operands; PDEFA_IO_SLICES=n: n, up to
+// kMatmulSlices.
 static int64_t matmul_slices(const MatmulLayout& L, int64_t M, int64_t K, int64_t N) {
+    if (const char* c = std::getenv("PDEFA_IO_SLICES"); c && std::atoi(c) > 0)
+        return std::min<int64_t>({kMatmulSlices, M, std::atoi(c)});
     return pipeline_slices(static_cast<double>(M * K) / kLinkFloatsPerUs, static_cast<double>(M * N) / kLinkFloatsPerUs,
                            std::min<int64_t>(kMatmulSlices, M / 256), [&](int64_t n) {
                                k::ConvArgs c;
@@ -2021,11 +2025,6 @@ static int64_t matmul_slices(const MatmulLayout& L, int64_t M, int64_t K, int64_
                                c.splits = L.ls.splits;
                                return launch_us(c, L.ls.tile) * static_cast<double>(n);
                            });
-}
-
-int64_t matmul_slices(int64_t M, int64_t K, int64_t N) {
-    if (M <= 0 || K <= 0 || N <= 0) return 1;
-    return matmul_slices(matmul_layout(M, K, N), M, K, N);
 }
 
 void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {

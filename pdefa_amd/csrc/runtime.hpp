@@ -287,9 +287,6 @@ struct MatmulHost {
 // C = A @ B on the device (the ops_matmul path).
 void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N);
 
-// Row slices that device_matmul cuts a product of page-locked operands into.
-int64_t matmul_slices(int64_t M, int64_t K, int64_t N);
-
 // The same product with its device buffers (A, B, packed B, bias, C, split-K
 // partials) in the static scratch array instead of allocated memory; throws
 // std::invalid_argument when they do not fit it.  Calls in one process are

@@ -72,7 +72,6 @@ def lib() -> C.CDLL:
             "pdefa_amd_plan_model": (C.c_int, [vp, C.POINTER(i64), i32, C.c_char_p, sz, C.POINTER(sz)]),
             "pdefa_amd_device_name": (C.c_char_p, []),
             "pdefa_amd_tune_stats": (C.c_int, [C.POINTER(i64), C.POINTER(i64)]),
-            "pdefa_amd_matmul_slices": (C.c_int, [i64, i64, i64, C.POINTER(i64)]),
             "pdefa_amd_pack_cache_stats": (C.c_int, [C.POINTER(i64), C.POINTER(i64)]),
             "pdefa_amd_ops_matmul_noalloc": (C.c_int, [vp, vp, vp]),
             "pdefa_amd_session_read_conv_input": (C.c_int, [vp, C.c_char_p, C.POINTER(C.c_float), sz,

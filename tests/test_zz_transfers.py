@@ -3,7 +3,6 @@ sliced runs (PDEFA_IO_SLICES) give the bits of the same program run without
 either (PDEFA_HIP_GRAPH=0: upload, every step, download).  The products here
 grow ops_matmul's scratch, so this file runs after test_zz_no_alloc, which
 watches it grow."""
-import ctypes as C
 import os
 import re
 
@@ -84,22 +83,14 @@ def test_block_transfers(kind, c, h, w, batch, tmp_path, monkeypatch):
     _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8], "batch", batch, True)
 
 
-def _matmul_slices(m, k, n):
-    out = C.c_int64()
-    native.check(native.lib().pdefa_amd_matmul_slices(m, k, n, C.byref(out)), "pdefa_amd_matmul_slices")
-    return out.value
-
-
 # Row counts around the slice rule's smallest slice, a remainder row per slice,
 # K % 4 != 0 (4-byte operand loads), products below and above the sizes from
 # which operands are page-locked and sliced, and C in A's memory (never sliced).
-@pytest.mark.parametrize("m,k,n,slices", [(1, 5, 7, 1), (300, 260, 300, 1), (512, 512, 512, 1), (2049, 1023, 1030, 3),
-                                          (3001, 2047, 601, 2), (3001, 2047, 1733, 4)])
-def test_matmul_transfers(m, k, n, slices):
+@pytest.mark.parametrize("m,k,n", [(1, 5, 7), (300, 260, 300), (512, 512, 512), (2049, 1023, 1030), (3001, 2047, 601)])
+def test_matmul_transfers(m, k, n):
     from pdefa_amd import pdefa as api
 
     print(f"[case] matmul {m}x{k}x{n}", flush=True)
-    assert _matmul_slices(m, k, n) == slices
     rng = np.random.default_rng(7)
     for _ in range(2):
         a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
@@ -110,6 +101,23 @@ def test_matmul_transfers(m, k, n, slices):
         # k products of unit variance, each partial sum rounded to 2^-24 of
         # itself: an error of about sqrt(k) * sqrt(k) * 2^-24 at the most
         np.testing.assert_allclose(out.numpy(), want, rtol=0, atol=k * 2.0**-24 * 4 + 1e-6)
+
+
+@pytest.mark.parametrize("m,k,n", [(258, 260, 300), (513, 512, 512), (2049, 1023, 1030)])
+def test_matmul_slices(m, k, n, monkeypatch):
+    """Every number of row slices (operands that are page-locked, in memory of
+    their own: the count asked for is the one that runs) gives the whole
+    product's bits."""
+    print(f"[case] matmul slices {m}x{k}x{n}", flush=True)
+    assert min(m * k, k * n, m * n) * 4 >= 256 * 1024  # page-locked
+    rng = np.random.default_rng(7)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    outs = []
+    for slices in (1, 2, 3, 4):
+        monkeypatch.setenv("PDEFA_IO_SLICES", str(slices))
+        outs.append(native.matmul(a, b))
+    for out in outs[1:]:
+        np.testing.assert_array_equal(out, outs[0])
 
 
 def test_matmul_of_many_rows():
