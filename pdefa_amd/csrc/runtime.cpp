@@ -1653,7 +1653,13 @@ void Session::run() {
         const char* h = reinterpret_cast<const char*>(prep_->host_out[0]);
         return a < h + prep_->outputs[0].nbytes && h < a + inputs_[0]->nbytes;
     };
-    const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged() && !in_output();
+    // (slices of output rows take page-locked inputs: their uploads are pitched
+    // copies, which the runtime stages row by row from pageable memory, 64 ->
+    // 64 3x3 at 160x160 1427 us against 379 unsliced, 128 -> 64 1x1 2708
+    // against 541; slices of the batch are whole runs, YOLOv8m C2f at 40x40,
+    // batch 16, 2540 against 2675)
+    const bool io = !segmented && !per_step && !prep_->io.empty() && !has_staged() && !in_output() &&
+                    (prep_->io.front().up.rows <= 1 || inputs_[0]->pinned);
     last_io_ = io ? static_cast<int32_t>(prep_->io.size()) : 0;
     if (!segmented && !io) upload_inputs();  // run_segments uploads (by slices) itself
     if (per_step) {

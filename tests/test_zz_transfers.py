@@ -55,7 +55,8 @@ def _check(model, shape, tmp_path, monkeypatch, slices, kind, most, direct):
         assert f"transfers pull=1 push=1 slices={kind}\n" in plan
         ran, pull, push, last = map(int, re.search(
             r"io slices=(\d+) pull_direct=(\d) push_direct=(\d) last_run=(\d+)", plan).groups())
-        assert last == ran
+        # slices of rows take page-locked inputs
+        assert last == (ran if ran == 1 or kind == "batch" or xs[0].nbytes >= 256 * 1024 else 0)
         if s:
             assert ran == (1 if kind == "none" else max(1, min(s, most)))
         assert (pull, push) == (int(direct and ran == 1),) * 2
@@ -69,7 +70,7 @@ def _check(model, shape, tmp_path, monkeypatch, slices, kind, most, direct):
 # which host tensors are page-locked.
 @pytest.mark.parametrize("cin,cout,k,s,hw", [
     (64, 64, 3, 1, 40), (32, 66, 3, 1, 37), (16, 24, 3, 2, 65), (96, 144, 3, 2, 33), (64, 65, 1, 1, 50),
-    (128, 64, 1, 1, 31), (16, 16, 3, 1, 16), (24, 40, 3, 2, 18),
+    (128, 64, 1, 1, 31), (16, 16, 3, 1, 16), (24, 40, 3, 2, 18), (32, 66, 3, 1, 61), (64, 30, 3, 2, 43),
 ])
 def test_single_conv_transfers(cin, cout, k, s, hw, tmp_path, monkeypatch):
     model = ys.build_single_conv(cin, cout, k, s, hw, seed=3)[0]
@@ -77,10 +78,27 @@ def test_single_conv_transfers(cin, cout, k, s, hw, tmp_path, monkeypatch):
 
 
 @pytest.mark.parametrize("kind,c,h,w,batch", [
-    ("c2f", 64, 20, 24, 5), ("c2f", 96, 13, 11, 2), ("sppf", 64, 21, 20, 3), ("scdown", 64, 22, 22, 4),
+    ("c2f", 64, 20, 24, 5), ("c2f", 96, 13, 11, 2), ("c2f", 96, 37, 31, 3), ("sppf", 64, 21, 20, 3), ("scdown", 64, 22, 22, 4),
 ])
 def test_block_transfers(kind, c, h, w, batch, tmp_path, monkeypatch):
     _check(_block(kind, c, h, w, batch), (batch, c, h, w), tmp_path, monkeypatch, [0, 1, 2, 3, 8], "batch", batch, True)
+
+
+@pytest.mark.parametrize("name,pinned", [("pageable", False), ("page-locked", True)])
+def test_row_slices_need_page_locked_inputs(name, pinned, tmp_path):
+    """A pageable input (under the size from which tensors are page-locked
+    here) goes up whole, whatever the slices asked for."""
+    model = ys.build_single_conv(16, 64, 3, 1, 80 if pinned else 60, seed=3)[0]
+    hw = 80 if pinned else 60
+    assert (16 * hw * hw * 4 >= 256 * 1024) == pinned
+    path = os.path.join(tmp_path, "m.engine")
+    ys.save(model, path)
+    x = np.random.default_rng(5).standard_normal((1, 16, hw, hw), dtype=np.float32)
+    want = _run(path, [x], {"PDEFA_HIP_GRAPH": "0"}, pytest.MonkeyPatch())[0]
+    got, plan = _run(path, [x], {"PDEFA_IO_SLICES": "3"}, pytest.MonkeyPatch())
+    print(f"[case] {name}", flush=True)
+    assert "io slices=3 " in plan and f" last_run={3 if pinned else 0}\n" in plan
+    np.testing.assert_array_equal(got[0], want[0])
 
 
 # Row counts around the slice rule's smallest slice, a remainder row per slice,
