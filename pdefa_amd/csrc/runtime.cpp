@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <sstream>
@@ -383,6 +384,30 @@ std::shared_ptr<DeviceModel> device_model(Model& m) {
 
 // ------------------------------------------------------------------ Session
 
+namespace {
+
+// Where a scope is left by an exception, the work on these streams (those that
+// exist by then) is waited for: copies in flight would go on reading and
+// writing tensors that the caller may free, and buffers that the next call
+// fills.
+class DrainOnThrow {
+   public:
+    DrainOnThrow(hipStream_t& a, hipStream_t& b, hipStream_t& c) : s_{&a, &b, &c}, thrown_(std::uncaught_exceptions()) {}
+    DrainOnThrow(const DrainOnThrow&) = delete;
+    DrainOnThrow& operator=(const DrainOnThrow&) = delete;
+    ~DrainOnThrow() {
+        if (std::uncaught_exceptions() == thrown_) return;
+        for (hipStream_t* s : s_)
+            if (*s) (void)hipStreamSynchronize(*s);
+    }
+
+   private:
+    hipStream_t* s_[3];
+    int thrown_;
+};
+
+}  // namespace
+
 Session::Session(Model& m) : model_(&m) {
     inputs_.assign(static_cast<size_t>(m.num_inputs()), nullptr);
     use_graph_ = env_flag("PDEFA_HIP_GRAPH", true);
@@ -584,6 +609,7 @@ std::vector<LetterboxGeometry> Session::set_images(int32_t idx, const std::vecto
     st.scale = scale;
     st.pad = pad;
     std::vector<LetterboxGeometry> geo;
+    std::vector<StagedImage> staged;  // all of them or, if a copy fails, none
     size_t off = 0;
     for (const ImageRef& im : images) {
         const size_t n = static_cast<size_t>(im.width) * im.height * im.channels;
@@ -595,10 +621,11 @@ std::vector<LetterboxGeometry> Session::set_images(int32_t idx, const std::vecto
         si.img = im;
         si.img.pixels = nullptr;
         si.g = letterbox_geometry(im.width, im.height, tw, th);
-        st.images.push_back(si);
+        staged.push_back(si);
         geo.push_back(si.g);
         off = (off + n + 255) / 256 * 256;
     }
+    st.images = std::move(staged);
     inputs_[idx] = nullptr;
     return geo;
 }
@@ -1644,6 +1671,7 @@ void Session::run() {
     if (!dev_) dev_ = device_model(*model_);
     if (!stream_) PDEFA_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     if (!prep_ || prep_->plan.input_dims != dims) prepare(dims);
+    DrainOnThrow drain(stream_, copy_in_, copy_out_);
     const bool per_step = prof_fn_ != nullptr || std::getenv("ENGINE_PROFILE_CSV") != nullptr;
     const bool segmented = use_graph_ && !per_step && !prep_->segments.empty();
     // (an input that lies in the memory of this run's output, the last run's
@@ -2051,6 +2079,7 @@ void device_matmul(const MatmulHost& h, int64_t M, int64_t K, int64_t N) {
     // goes down while later slices of A go up)
     const bool apart = h.C + M * N <= h.A || h.A + M * K <= h.C;
     const int64_t slices = h.a_pinned && h.b_pinned && h.c_pinned && apart ? matmul_slices(L, M, K, N) : 1;
+    DrainOnThrow drain(sc.stream, sc.up, sc.down);
     if (slices > 1)
         matmul_sliced(L, sc, h, M, K, N, slices);
     else
