@@ -1976,7 +1976,10 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 
 // Host A, B in; host C out; the device buffers at `base` (L.total() floats).
 // Up to kKernelBytes a page-locked operand moves by a kernel of the stream
-// (kernels/relayout.hip), larger ones by DMA copies.
+// (kernels/relayout.hip), larger ones and pageable ones by copies.  The copies
+// go first: a pageable operand's copy behind the kernel waits for it (371 x
+// 201 by 201 x 55, whose A alone is page-locked: 57 us, 47 with B's copy
+// first, 55 with copies only).
 void matmul_on(const MatmulLayout& L, float* base, const MatmulHost& h, int64_t M, int64_t K, int64_t N,
                hipStream_t s) {
     constexpr int64_t kKernelBytes = 8 << 20;
@@ -1985,24 +1988,23 @@ void matmul_on(const MatmulLayout& L, float* base, const MatmulHost& h, int64_t 
     float* dP = dB + L.nB;
     float* dBias = dP + L.nP;
     float* dC = dBias + L.nBias;
-    auto move = [&](float* dst, const float* src, int64_t n, bool pinned, hipMemcpyKind kind) {
-        const int64_t bytes = static_cast<int64_t>(sizeof(float)) * n;
-        if (pinned && bytes <= kKernelBytes && aligned16(src) && aligned16(dst))
-            k::launch_copy_floats({{dst, src, n}}, s);
-        else
-            PDEFA_HIP(hipMemcpyAsync(dst, src, static_cast<size_t>(bytes), kind, s));
+    auto by_kernel = [](const float* host, int64_t n, bool pinned) {
+        return pinned && static_cast<int64_t>(sizeof(float)) * n <= kKernelBytes && aligned16(host);
     };
-    if (h.a_pinned && h.b_pinned && 4 * M * K <= kKernelBytes && 4 * K * N <= kKernelBytes && aligned16(h.A) &&
-        aligned16(h.B)) {
-        k::launch_copy_floats({{dA, h.A, M * K}, {dB, h.B, K * N}}, s);
-    } else {
-        move(dA, h.A, M * K, h.a_pinned, hipMemcpyHostToDevice);
-        move(dB, h.B, K * N, h.b_pinned, hipMemcpyHostToDevice);
-    }
+    auto copy = [&](float* dst, const float* src, int64_t n, hipMemcpyKind kind) {
+        PDEFA_HIP(hipMemcpyAsync(dst, src, sizeof(float) * static_cast<size_t>(n), kind, s));
+    };
+    const bool a_kernel = by_kernel(h.A, M * K, h.a_pinned), b_kernel = by_kernel(h.B, K * N, h.b_pinned);
+    if (!a_kernel) copy(dA, h.A, M * K, hipMemcpyHostToDevice);
+    if (!b_kernel) copy(dB, h.B, K * N, hipMemcpyHostToDevice);
+    k::launch_copy_floats({{dA, h.A, a_kernel ? M * K : 0}, {dB, h.B, b_kernel ? K * N : 0}}, s);
     k::launch_pack_gemm_b(dP, dB, static_cast<int>(K), static_cast<int>(N), dBias, s);
     matmul_rows(L, base, 0, M, K, N, s);
     PDEFA_HIP(hipGetLastError());
-    move(h.C, dC, M * N, h.c_pinned, hipMemcpyDeviceToHost);
+    if (by_kernel(h.C, M * N, h.c_pinned))
+        k::launch_copy_floats({{h.C, dC, M * N}}, s);
+    else
+        copy(h.C, dC, M * N, hipMemcpyDeviceToHost);
     PDEFA_HIP(hipStreamSynchronize(s));
 }
 

@@ -103,8 +103,10 @@ def test_row_slices_need_page_locked_inputs(name, pinned, tmp_path):
 
 # Row counts around the slice rule's smallest slice, a remainder row per slice,
 # K % 4 != 0 (4-byte operand loads), products below and above the sizes from
-# which operands are page-locked and sliced, and C in A's memory (never sliced).
-@pytest.mark.parametrize("m,k,n", [(1, 5, 7), (300, 260, 300), (512, 512, 512), (2049, 1023, 1030), (3001, 2047, 601)])
+# which operands are page-locked (each of A, B and C alone too) and sliced, and
+# C in A's memory (never sliced).
+@pytest.mark.parametrize("m,k,n", [(1, 5, 7), (300, 260, 300), (512, 512, 512), (2049, 1023, 1030), (3001, 2047, 601),
+                                   (371, 201, 55), (32, 1251, 211), (300, 100, 300), (64, 300, 2000), (1659, 69, 518)])
 def test_matmul_transfers(m, k, n):
     from pdefa_amd import pdefa as api
 
