@@ -420,8 +420,9 @@ __device__ __forceinline__ void conv_tile(const ConvArgs& a, const int bx, const
     // element, 7 for A's with the row magnitudes) and the CU 1400 of LDS
     // traffic, which overlap only in part (about 3800 measured).  16 x 40x40
     // images, us against the f32 tile of the launch-shape table: 768 -> 384
-    // 1x1 108 / 140 (210 TFLOP/s), 384 -> 384 1x1 66 / 79; 16 x 20x20, 1152
-    // -> 576: 63 / 85.  Tried, against 114 for the first of these with the
+    // 1x1 108 / 140 (140 TFLOP/s), 384 -> 384 1x1 66 / 79; 16 x 20x20, 1152
+    // -> 576: 63 / 85; 16 x 80x80, 192 -> 384 3x3 stride 2: 219 / 293 (155
+    // TFLOP/s).  Tried, against 114 for the first of these with the
     // infinities handled in truncated terms: four waves of 64x64 (140) and
     // 128 x 64 tiles, two workgroups a CU (124); one quarter's fragments at a
     // time (129); the groups of products held in order by scheduling barriers

@@ -1693,16 +1693,21 @@ class Planner {
 
     // Long implicit GEMMs to the split tile (PlanOptions::split_terms): those
     // whose output channels fill its 128-wide columns to 90%, whose tiles
-    // fill half the CUs and whose K is at least 768.  Measured on YOLOv8m's
-    // layers at batch 16 (us, the launch-shape table's f32 tile / split):
-    // with Cout 384 and 576, K from 384 to 3456 79 / 62 to 236 / 157 (1.28 to
-    // 1.51 times faster); with Cout 192 (75% of the columns) 1.04 to 1.12
-    // times faster at K 384 to 1728 and slower at 192, with Cout 96 1.07 at
-    // K 192 and slower at 96, with Cout 64 slower; 3x3 stride-1 layers
-    // stay with Winograd, 114 against 165.  The wide layers with K below 768
-    // are the entry convs of C2f blocks: their rounding decides which side of
-    // a SiLU jump some outputs of the 3x3 layers behind them take, and the 20
-    // us each would save are not worth moving those.
+    // fill half the CUs and whose K is at least 768.  Measured (us, the f32
+    // tile that the launch-shape table or a timing gives / split), YOLOv8m's
+    // layers at batch 16: Cout 384 and 576, K 768 to 3456 85 / 63 to 293 /
+    // 219 (1.30 to 1.38 times faster); Cout 192 (75% of the columns) 1.04 to
+    // 1.12 times faster at K 384 to 1728 and slower at 192, Cout 96 1.07 at K
+    // 192 and slower at 96, Cout 64 slower; 3x3 stride-1 layers stay with
+    // Winograd, 114 against 165.  By tiles, K 768 to 2304: 52 to 65 of them
+    // 0.54 to 0.57, 75 to 100 0.87 to 1.10, 125 1.08, 126 0.98 to 1.04, 150 to
+    // 250 1.16 to 1.45, 264 to 300 (a second round) 1.12 to 1.18.
+    // The count is the whole batch's; a program that runs in slices of it has
+    // fewer tiles a launch, with the f32 tile of the whole batch as well.
+    // The wide layers with K below 768 are the entry convs of C2f blocks: their
+    // rounding decides which side of a SiLU jump some outputs of the 3x3
+    // layers behind them take, and the 12 us each would save are not worth
+    // moving those.
     void split_long_gemms() {
         if (!opt_.split_terms) return;
         for (Step& s : plan_.steps) {

@@ -1377,19 +1377,24 @@ static double launch_us(const k::ConvArgs& c, int tile) {
     return 5.0 + flops / 1e8 / std::max(fill, 1e-3);
 }
 
-// The transfers of a sliced program are DMA copies on their own streams:
-// kernels that read or write host memory beside the steps' kernels hold those
-// up (a conv that takes 8 us alone took 41 beside a 41 us transfer kernel, on
-// 4 to 128 workgroups alike), the DMA engines do not.  With S slices the
-// upload, the steps and the download run side by side but for the first
-// slice's upload and the last one's rest, and each slice costs kSliceUs more
-// (copies wait for events, and events for copies, 15 to 35 us each); the
-// steps cost more too where a slice leaves the last round of workgroups
-// emptier (steps(S): their time in S slices).  S is the count up to `most`
-// with the least estimate; it is the measured best for the sizes tried (us
-// for S = 1, 2, 3, 4; YOLOv8m C2f at 40x40, batch 16: 2148, 1659, 1388, 1524;
-// its SPPF: 692, 588, 654, 747; 64 -> 64 3x3 at 160x160: 287, 266, 262, 267;
-// 128 -> 64 1x1: 396, 369, 370, 386) or within 2% of it.
+// The transfers of a sliced program are copies on their own streams: kernels
+// that read or write host memory beside the steps' kernels hold those up (a
+// conv that takes 8 us alone took 41 beside a 41 us transfer kernel, on 4 to
+// 128 workgroups alike), DMA copies do not.  (Contiguous downloads beside other
+// copies are the exception: in a trace the runtime does them by a kernel of its
+// own, and a slice's first conv takes 240 us beside one for 33 alone.)
+// With S slices the upload, the steps and the download run side by side but
+// for the first slice's upload and the last one's rest, and each slice costs
+// kSliceUs more (copies wait for events, and events for copies, 15 to 35 us
+// each); the steps cost more too where a slice leaves the last round of
+// workgroups emptier (steps(S): their time in S slices).  Each direction is
+// taken at its own 56 GB/s (both at once share 96).  S is the count up to
+// `most` with the least estimate.  Measured, us for S = 1, 2, 3, 4: YOLOv8m C2f
+// at 40x40, batch 16: 2148, 1659, 1388, 1524; its SPPF: 692, 588, 654, 747; 64
+// -> 64 3x3 at 160x160: 287, 266, 262, 267; 128 -> 64 1x1: 396, 369, 370, 386.
+// Those four set kSliceUs and the rate in launch_us; over 34 other convs and
+// blocks (24 to 512 channels, 10x23 to 152x152, batch 1 to 14) the pass is
+// within 3% of the best count's, and within 1% for 32 of them.
 static constexpr double kLinkFloatsPerUs = 14000.0;  // 56 GB/s
 template <typename F>
 static int64_t pipeline_slices(double up_us, double down_us, int64_t most, F&& steps) {
@@ -1409,8 +1414,11 @@ static int64_t pipeline_slices(double up_us, double down_us, int64_t most, F&& s
 
 // An unsliced program moves a tensor of up to kDirectBytes by the transfer
 // kernels themselves, on the session stream: they start and end with the
-// program's kernels, without a DMA copy's waits (96 -> 144 3x3 at 33x33: 62
-// -> 41 us; a pass of YOLOv8n b1, whose head is 2.8 MB: 561 -> 558).
+// program's kernels, without a copy's waits (us, by copies / by kernels: 96 ->
+// 144 3x3 at 33x33 62 / 41; YOLOv8n at batch 1 272 / 263 at 160x160, 562 / 554
+// at 640x640; SPPF of 256 channels, 4.9 MB each way, 251 / 243).  Above it the
+// gain is under 1% (13 MB each way 590 / 584), and for as long as such a
+// kernel runs it holds up other sessions' kernels.
 void Session::plan_io() {
     constexpr int64_t kDirectBytes = 8 << 20;
     constexpr int64_t kMaxIoSlices = 4;

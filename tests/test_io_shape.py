@@ -46,8 +46,8 @@ def _conv_conv(c, hw, rows):
     return _graph(build, (1, c, hw, hw), (1, c, rows, hw)), (1, c, hw, hw)
 
 
-def _one_conv(cin, cout, k, s, hw):
-    return ys.build_single_conv(cin, cout, k, s, hw, seed=3)[0], (1, cin, hw, hw)
+def _one_conv(cin, cout, k, s, hw, groups=1):
+    return ys.build_single_conv(cin, cout, k, s, hw, seed=3, groups=groups)[0], (1, cin, hw, hw)
 
 
 def _batch(build, n, c, h, w, out_shape):
@@ -115,6 +115,10 @@ def _view_concat(n, c, h, w, view):
 CASES = {
     "conv": (lambda: _one_conv(64, 64, 3, 1, 48), "rows"),
     "conv 1x1": (lambda: _one_conv(32, 24, 1, 1, 40), "rows"),
+    "conv 5x5": (lambda: _one_conv(32, 40, 5, 1, 57), "rows"),
+    "conv 5x5 s2": (lambda: _one_conv(32, 40, 5, 2, 57), "rows"),
+    "conv in groups": (lambda: _one_conv(64, 64, 3, 1, 47, groups=4), "rows"),
+    "depthwise conv": (lambda: _one_conv(64, 64, 3, 1, 47, groups=64), "none"),
     # the last copy reads a part of the conv's rows, columns or channels
     "conv rows 4..48": (lambda: _conv_slice(64, 64, 3, 48, 2, 4, 48), "none"),
     "conv rows 0..24": (lambda: _conv_slice(64, 64, 3, 48, 2, 0, 24), "none"),
