@@ -443,7 +443,9 @@ PDEFA_EXPORT EngineStatus pdefa_amd_plan_model(const EngineModel* m, const int64
                                                std::vector<int64_t>(shape, shape + ndim));
         pdefa::PlanOptions opt;
         if (const char* r = std::getenv("PDEFA_REUSE_MEMORY")) opt.reuse_memory = r[0] != '0';
-        // as a session plans it: the Detect decode split per anchor range
+        // as a session plans it: the edges' copies in memory of their own, the
+        // Detect decode split per anchor range
+        opt.pin_io = true;
         const char* so = std::getenv("PDEFA_SPLIT_OUTPUTS");
         opt.split_outputs = !(so && so[0] == '0');
         // PDEFA_EARLY_HW, where it is set, as a session on a batch takes it

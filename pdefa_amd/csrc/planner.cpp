@@ -2099,6 +2099,7 @@ std::string describe_plan(const Model& m, const Plan& p) {
         os << " out=" << fmt_view(s.out) << " a=" << fmt_view(s.a);
         if ((s.kind == StepKind::Elt && s.elt >= k::kEltAdd && s.elt <= k::kEltDiv) || s.kind == StepKind::GatherElements)
             os << " b=" << fmt_view(s.b);
+        if (s.kind == StepKind::MaxPoolChain) os << " b=" << fmt_view(s.b) << " c=" << fmt_view(s.c);
         if (s.kind == StepKind::TopK)
             os << " axis=" << s.axis << " k=" << s.topk << (s.topk_indices ? " indices" : " values");
         if (s.kind == StepKind::GatherElements) os << " axis=" << s.axis;

@@ -2,6 +2,7 @@
 io_shape, printed with the plan): on the host by the plan text, and on the GPU
 by their outputs against the same program run without either."""
 import os
+import random
 import re
 
 import numpy as np
@@ -223,3 +224,126 @@ def test_outputs(name, tmp_path, monkeypatch):
         print(f"[case] {name} {env}", flush=True)
         for g, w in zip(_run(path, xs + xs[:1], env, monkeypatch), want + want[:1]):
             np.testing.assert_array_equal(g, w)
+
+
+# ---- the rules against what the steps do: random graphs, sliced on paper
+
+_VIEW = re.compile(r" (out|a|b|c|res|up)=b(-?\d+)\+(\d+)\[([\d,]*)\]s\[([-\d,]*)\]")
+
+
+def _views(line):
+    """(views read, views written) of a plan's step line: (buffer, offset, dims, strides)."""
+    writes = ("out", "b", "c") if " maxpool_chain " in line else ("out", "up")
+    rd, wr = [], []
+    for key, buf, off, dims, strides in _VIEW.findall(line):
+        v = (int(buf), int(off), [int(d) for d in dims.split(",")], [int(s) for s in strides.split(",")])
+        if v[0] >= 0:  # not a constant
+            (wr if key in writes else rd).append(v)
+    return rd, wr
+
+
+def _item(v, i):
+    """Elements of item i of a view's outer dimension."""
+    _, off, dims, strides = v
+    e = np.array([off + i * strides[0]])
+    for d, s in zip(dims[1:], strides[1:]):
+        e = (e[:, None] + np.arange(d) * s).reshape(-1)
+    return e
+
+
+def _run_sliced(steps, n, slices, inputs, elems):
+    """Runs steps slice by slice on tags: which image's data an element holds."""
+    mem = {inputs: np.full(elems, -1)}
+
+    def tags(v, e):
+        if v[0] not in mem or len(mem[v[0]]) <= e.max():
+            mem[v[0]] = np.concatenate([mem.get(v[0], np.empty(0, int)), np.full(int(e.max()) + 1, -1)])
+        return mem[v[0]]
+
+    for lo, hi in slices:
+        mem[inputs][lo * elems // n:hi * elems // n] = np.repeat(np.arange(lo, hi), elems // n)
+        for line in steps:
+            rd, wr = _views(line)
+            for i in range(lo, hi):
+                for v in rd:
+                    e = _item(v, i)
+                    assert (tags(v, e)[e] == i).all(), (line, i)
+            for i in range(lo, hi):
+                for v in wr:
+                    e = _item(v, i)
+                    tags(v, e)[e] = i
+
+
+def _random_graph(rng):
+    """A chain of convs, pools, views, concats and upsamples whose dimensions
+    often have the batch's size."""
+    n = rng.choice([2, 2, 4])
+    d = shape = [n, rng.choice([n, 4, 8, 16]), rng.choice([n, 4, 6]), rng.choice([n, 4, 5])]
+    b = ys.GraphBuilder()
+    y = ys._Yolo(b, np.random.default_rng(1), 0.0)
+    x, old = -1, []
+    for i, op in enumerate(["conv"] * (rng.random() < 0.7) + rng.choices(
+            ["conv", "conv s2", "pool", "slice", "reshape", "transpose", "concat", "resize"], k=rng.randint(1, 4))):
+        d = list(d)
+        if op.startswith("conv"):
+            c, s = rng.choice([8, 16, 8 * n]), 2 if op == "conv s2" else 1
+            x = y.conv(x, d[1], c, rng.choice([1, 3]) if s == 1 else 3, s, f"c{i}")
+            d = [d[0], c, (d[2] - 1) // s + 1, (d[3] - 1) // s + 1]
+        elif op == "pool":
+            x = b.node("MaxPool", f"/p{i}", [x], kernel_h=3, kernel_w=3, stride_h=1, stride_w=1, pad_h=1, pad_w=1)
+        elif op == "slice":
+            ax = rng.randrange(4)
+            size = n if d[ax] > n and rng.random() < 0.5 else rng.randint(1, d[ax])
+            lo = rng.randint(0, d[ax] - size)
+            x, d[ax] = y.slice(x, lo, lo + size, ax, f"/s{i}"), size
+        elif op == "reshape":
+            p, q = rng.sample(range(4), 2)
+            if d[p] % 2 == 0:
+                d[p], d[q] = d[p] // 2, d[q] * 2
+                x = b.node("Reshape", f"/r{i}", [x, b.const(f"/r{i}::shape", d)])
+        elif op == "transpose":
+            perm = rng.sample(range(4), 4)
+            x, d = b.node("Transpose", f"/t{i}", [x, b.const(f"/t{i}::perm", np.array(perm, np.float32))]), [d[p] for p in perm]
+        elif op == "concat":
+            other = [o for o in old if o[1][0] == d[0] and o[1][2:] == d[2:]]
+            k, c = rng.choice(other) if other else (b.const(f"/k{i}", np.ones((d[0], 4, d[2], d[3]))), [0, 4])
+            x, d[1] = b.node("Concat", f"/cat{i}", [x, k], axis=1), d[1] + c[1]
+        else:
+            x, d = y.upsample(x, f"u{i}"), [d[0], d[1], 2 * d[2], 2 * d[3]]
+        old.append((x, d))
+    return b.model(shape, d, [x]), shape
+
+
+def test_random_graphs(tmp_path, monkeypatch):
+    """Every step of a program that runs in slices of the batch, or early on
+    chunks of it, reads only what its own slice has written."""
+    monkeypatch.setenv("PDEFA_EARLY_HW", "1")
+    path = os.path.join(tmp_path, "m.engine")
+    batch = early = 0
+    for seed in range(600):
+        model, shape = _random_graph(random.Random(seed))
+        if not model.nodes:
+            continue
+        ys.save(model, path)
+        try:
+            text = native.plan_text(path, shape)
+        except native.NativeError:
+            continue  # a form that the device program does not take
+        steps = text.split("\narena")[0].splitlines()[1:]
+        if not steps:
+            continue
+        n, elems = shape[0], int(np.prod(shape))
+        written = {v[0] for line in steps for v in _views(line)[1]}
+        inputs = {v[0] for line in steps for v in _views(line)[0]} - written
+        if len(inputs) != 1:
+            continue
+        inputs = inputs.pop()
+        if transfers(text)[2] == "batch":
+            batch += 1
+            for s in {2, n}:
+                _run_sliced(steps, n, [(n * i // s, n * (i + 1) // s) for i in range(s)], inputs, elems)
+        e = int(re.search(r"early_steps=(\d+)", text).group(1))
+        if e:
+            early += 1
+            _run_sliced(steps[:e], n, [(0, n // 2), (n // 2, n)], inputs, elems)
+    assert batch > 60 and early > 200
