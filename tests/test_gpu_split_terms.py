@@ -214,3 +214,51 @@ def test_split_tile_single_products(x_bits, tmp_path, monkeypatch):
     # centred: over random significands the mean error is far below the largest
     if x_bits is None:
         assert abs((rel * np.sign(want)).mean()) <= 2.0**-29
+
+
+def test_split_tile_compat_silu(tmp_path, monkeypatch):
+    """A 3x3 stride-1 layer (the SiLU form with the float64 second pass) on
+    the split tile: an infinity and a pixel of tiny values in one tile each
+    give the f32 tile's bits there, other tiles the split sums."""
+    print("[case] split compat SiLU", flush=True)
+    path = _engine(ys.build_single_conv(64, 128, 3, 1, 24, seed=3)[0], os.path.join(tmp_path, "c.engine"))
+    x = np.random.default_rng(2).standard_normal((1, 64, 24, 24)).astype(np.float32)
+    plain = [_run(path, x, t, monkeypatch) for t in ("split128x128w8", "128x128w8")]
+    # a SiLU jump of 2% lies between the two sums at a few outputs at most
+    off = np.abs(plain[0] - plain[1]) > 1e-4 * (1 + np.abs(plain[1]))
+    assert off.sum() <= 3
+    x[0, 5, 1, 1] = np.inf
+    got, f32 = (_run(path, x, t, monkeypatch) for t in ("split128x128w8", "128x128w8"))
+    # the first tile: output rows 0 to 4 and 8 pixels of row 5
+    np.testing.assert_array_equal(got[:, :, :5], f32[:, :, :5])
+    assert not np.array_equal(got[:, :, 6:], f32[:, :, 6:])
+
+
+def test_split_tile_upsampled_copy(tmp_path, monkeypatch):
+    """A layer that the rule takes and whose epilogue writes an upsampled copy,
+    with a NaN in one tile."""
+    print("[case] split upsampled copy", flush=True)
+    b = ys.GraphBuilder()
+    y = ys._Yolo(b, np.random.default_rng(3), 0.0)
+    out = y.conv(y.upsample(y.conv(-1, 768, 128, 1, 1, "c"), "u"), 128, 16, 1, 1, "d")
+    path = _engine(b.model([1, 768, 128, 128], [1, 16, 256, 256], [out]), os.path.join(tmp_path, "c.engine"))
+    x = np.random.default_rng(2).standard_normal((1, 768, 128, 128)).astype(np.float32)
+    x[0, 700, 3, 77] = np.nan
+    outs = []
+    for terms in ("1", "0"):
+        monkeypatch.setenv("PDEFA_SPLIT_TERMS", terms)
+        eng = native.Engine(path)
+        try:
+            outs.append(eng.run(x)[0].copy())
+            conv = next(l for l in eng.plan().splitlines() if " conv_mfma(" in l)
+        finally:
+            eng.close()
+        assert ("tile=split128x128w8" in conv) == (terms == "1") and " up=b" in conv
+    got, f32 = outs
+    nan = np.zeros((256, 256), bool)
+    nan[6:8, 154:156] = True
+    np.testing.assert_array_equal(np.isnan(got[0]), np.broadcast_to(nan, got[0].shape))
+    np.testing.assert_array_equal(np.isnan(f32), np.isnan(got))
+    # 768 and 128 products of about unit size, in sums of either order, each
+    # addition rounded to 2^-24 of a few units
+    np.testing.assert_allclose(got[~np.isnan(got)], f32[~np.isnan(f32)], rtol=1e-5, atol=(768 + 128) * 2.0**-24)
